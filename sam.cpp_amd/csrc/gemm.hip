@@ -15,6 +15,47 @@ namespace {
 constexpr int BM = 128, BN = 128, BK = 32;
 constexpr int LDS_STRIDE = BK + 8;   // halves; 80-byte rows keep 16-byte reads conflict-free
 constexpr int GROUP_M = 8;
+// The 16 weights of one thread and K step between their load and their
+// decoding.  WeightPiece aligns the bytes as part of the load, which waits
+// for them; Q8_0 rows (the ones this kernel gets by default) keep the dwords
+// as they were read, so that DEPTH steps of loads can be in flight.
+template <int WT> struct StepPiece : WeightPiece<WT> {
+    __device__ __forceinline__ void load_step(const uint8_t* row, int step, int h) { this->load(row, step, h); }
+    __device__ __forceinline__ void decode(const uint8_t*, int step, int h, _Float16* out) const {
+        this->dequant(step, h, out);
+    }
+};
+template <> struct StepPiece<T_Q8_0> {
+    uint32_t w[5], d;
+    // byte (0 or 2) at which the step's block starts in its first dword
+    static __device__ __forceinline__ uint32_t shift(const uint8_t* row, int step) {
+        return uint32_t(reinterpret_cast<uintptr_t>(row) + 34 * step) & 2;
+    }
+    __device__ __forceinline__ void load_step(const uint8_t* row, int step, int h) {
+        const uint32_t sd = shift(row, step), sc = sd ^ 2;   // the codes start two bytes on
+        const uint8_t* blk = row + 34 * step;
+        d = *reinterpret_cast<const uint32_t*>(blk - sd);
+        const uint32_t* q = reinterpret_cast<const uint32_t*>(blk + 2 + 16 * h - sc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = q[i];
+        w[4] = q[sc ? 4 : 3];   // no dword without one of the 16 bytes is touched
+    }
+    __device__ __forceinline__ void decode(const uint8_t* row, int step, int, _Float16* out) const {
+        const uint32_t sd = shift(row, step), sc = sd ^ 2;
+        const _Float16 dh = __builtin_bit_cast(_Float16, uint16_t(sd ? d >> 16 : d));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mul_i8x4_to_half(funnel_bytes(w[i + 1], w[i], sc), dh, out + 4 * i);
+    }
+};
+
+// K steps in flight per thread, in registers.  A tile has its CU to itself
+// when the grid is small, and one step's products (8 MFMAs a wave) are far
+// shorter than the latency of its scattered packed-weight loads: M = 300,
+// N = 259, K = 800 (9 tiles) 35.1 -> 25.6 us with its staging, M = 1000,
+// N = 1000, K = 4064 (64 tiles) 138 -> 77; grids of many tiles are level
+// (M = 20000, N = 3000, K = 800 218 -> 222).
+template <int WT>
+constexpr int kDepth = WT == T_Q8_0 ? 4 : 2;
 
 // Tile order: blocks are dispatched round-robin over the 8 XCDs, so give each
 // XCD a contiguous range of tiles, and walk that range in groups of GROUP_M
@@ -38,6 +79,8 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const _Float16* __restrict
                                                       const uint8_t* __restrict__ W, int64_t w_stride,
                                                       float* __restrict__ Y, int64_t ldy, int M, int N, int K,
                                                       int tiles_m, int tiles_n) {
+    constexpr int DEPTH = kDepth<WT>;
+    static_assert(DEPTH % 2 == 0, "the LDS buffer alternates per step");
     __shared__ _Float16 As[2][BM * LDS_STRIDE];
     __shared__ _Float16 Bs[2][BN * LDS_STRIDE];
 
@@ -49,54 +92,46 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const _Float16* __restrict
     const int wm = wave >> 1, wn = wave & 1;
     // loader role: row lr of the tile, 16-element half lh of the K step
     const int lr = tid >> 1, lh = tid & 1;
-    const bool a_ok = m0 + lr < M;
-    const bool b_ok = n0 + lr < N;
-    const _Float16* a_src = A + int64_t(a_ok ? m0 + lr : 0) * lda + 16 * lh;
-    const uint8_t* w_row = W + int64_t(b_ok ? n0 + lr : 0) * w_stride;
+    // rows past M or N repeat the last one; their products are not stored
+    const _Float16* a_src = A + int64_t(min(m0 + lr, M - 1)) * lda + 16 * lh;
+    const uint8_t* w_row = W + int64_t(min(n0 + lr, N - 1)) * w_stride;
 
     floatx16 acc[2][2];
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j)
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    u32x4 a_reg[2];
-    WeightPiece<WT> b_reg;
+    u32x4 a_reg[DEPTH][2];
+    StepPiece<WT> b_reg[DEPTH];
 
-    auto global_load = [&](int step) {
-        if (a_ok) {
-            const u32x4* p = reinterpret_cast<const u32x4*>(a_src + BK * step);
-            a_reg[0] = p[0];
-            a_reg[1] = p[1];
-        } else {
-            a_reg[0] = u32x4{0, 0, 0, 0};
-            a_reg[1] = u32x4{0, 0, 0, 0};
-        }
-        if (b_ok) b_reg.load(w_row, step, lh);
+    const int nsteps = K / BK;
+    auto global_load = [&](int slot, int step) {
+        const int st = min(step, nsteps - 1);   // past the range: a repeat of the last step, never stored to LDS
+        const u32x4* p = reinterpret_cast<const u32x4*>(a_src + BK * st);
+        a_reg[slot][0] = p[0];
+        a_reg[slot][1] = p[1];
+        b_reg[slot].load_step(w_row, st, lh);
     };
-    auto lds_store = [&](int buf, int step) {
+    auto lds_store = [&](int buf, int slot, int step) {
         u32x4* ad = reinterpret_cast<u32x4*>(&As[buf][lr * LDS_STRIDE + 16 * lh]);
-        ad[0] = a_reg[0];
-        ad[1] = a_reg[1];
+        ad[0] = a_reg[slot][0];
+        ad[1] = a_reg[slot][1];
         _Float16 w[16];
-        if (b_ok) {
-            b_reg.dequant(step, lh, w);
-        } else {
-            for (int i = 0; i < 16; ++i) w[i] = (_Float16)0.f;
-        }
+        b_reg[slot].decode(w_row, step, lh, w);
         half8* bd = reinterpret_cast<half8*>(&Bs[buf][lr * LDS_STRIDE + 16 * lh]);
         bd[0] = half8{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
         bd[1] = half8{w[8], w[9], w[10], w[11], w[12], w[13], w[14], w[15]};
     };
 
-    const int nsteps = K / BK;
-    global_load(0);
-    lds_store(0, 0);
+    // slot i of the register ring holds a step s with s % DEPTH == i
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) global_load(i, i);
+    lds_store(0, 0, 0);
+    global_load(0, DEPTH);
     __syncthreads();
 
     const int frag_row = lane & 31, frag_k = 8 * (lane >> 5);
-    for (int s = 0; s < nsteps; ++s) {
-        const int buf = s & 1;
-        if (s + 1 < nsteps) global_load(s + 1);
+    auto products = [&](int buf) {
 #pragma unroll
         for (int ks = 0; ks < BK; ks += 16) {
             half8 af[2], bf[2];
@@ -112,7 +147,25 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const _Float16* __restrict
                 for (int j = 0; j < 2; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
         }
-        if (s + 1 < nsteps) lds_store(buf ^ 1, s + 1);
+    };
+    // whole turns of the ring without a branch, so that each wait counts
+    // exactly the loads issued since; then the up to DEPTH - 1 steps left
+    int s0 = 0;
+    for (; s0 + DEPTH <= nsteps; s0 += DEPTH) {
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u) {
+            const int next = (u + 1) % DEPTH;
+            products(u & 1);
+            lds_store((u & 1) ^ 1, next, min(s0 + u + 1, nsteps - 1));
+            global_load(next, s0 + u + 1 + DEPTH);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < DEPTH - 1; ++u) {
+        if (s0 + u >= nsteps) break;
+        products(u & 1);
+        if (s0 + u + 1 < nsteps) lds_store((u & 1) ^ 1, u + 1, s0 + u + 1);
         __syncthreads();
     }
 
