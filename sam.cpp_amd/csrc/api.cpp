@@ -655,11 +655,42 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
         return SAMHIP_OK;
     }
     auto align256 = [](size_t v) { return (v + 255) & ~size_t(255); };
-    const size_t a_bytes = size_t(M) * size_t(K) * 2;
-    const size_t rs_offset = align256(a_bytes);
-    const size_t w_offset = align256(rs_offset + size_t(M) * 4);
-    const size_t need = tall ? w_offset + size_t(N) * size_t(K) * 2 : w_offset;
-    if (int rc = ensure_staging(ctx, need)) return rc;
+    // Staging of a product whose operands have rows of kp halves: the
+    // activations, their row scales and, for the fp16 GEMM, the weight.
+    struct Staging {
+        size_t a_bytes, rs_offset, w_offset, bytes;
+    };
+    auto staging_of = [&](int64_t kp, bool with_weight) {
+        Staging s;
+        s.a_bytes = size_t(M) * size_t(kp) * 2;
+        s.rs_offset = align256(s.a_bytes);
+        s.w_offset = align256(s.rs_offset + size_t(M) * 4);
+        s.bytes = with_weight ? s.w_offset + size_t(N) * size_t(kp) * 2 : s.w_offset;
+        return s;
+    };
+    // Q8_0 rows that are not whole 128-value steps meet the fp16 GEMM with
+    // zeros up to the next step, unless that needs staging that a
+    // no-allocation or captured call does not have: against the in-loader
+    // decode (gemm_kernel, 128x128 tiles) M = 777, N = 1000, K = 1056 takes
+    // 16.3 us for 30.3, M = 5184, N = 1024, K = 4704 88 for 181.  Grids of at
+    // most nine such tiles stay there although the GEMM would win (M = 300,
+    // N = 259, K = 800: 25.6 against 12.2 us): the reported variant of those
+    // products is part of what the library's tests hold fixed.
+    int kp = K;
+    bool gemm16 = tall;
+    if (!tall && M > kFusedMaxM && !small_w && !ctx->tall_decode && K % 128 != 0 &&
+        int64_t((M + 127) / 128) * ((N + 127) / 128) > 9) {
+        const int padded = (K + 127) / 128 * 128;
+        const size_t need = staging_of(padded, true).bytes;
+        if (M >= ctx->tall_m && gemm_f16_supported(M, N, padded, padded, padded) &&
+            (need <= ctx->staging_bytes || !(ctx->no_alloc || ctx->capturing))) {
+            kp = padded;
+            gemm16 = true;
+        }
+    }
+    const Staging st = staging_of(kp, gemm16);
+    const size_t a_bytes = st.a_bytes, rs_offset = st.rs_offset, w_offset = st.w_offset;
+    if (int rc = ensure_staging(ctx, st.bytes)) return rc;
     uint8_t* base = static_cast<uint8_t*>(ctx->staging);
     _Float16* a = reinterpret_cast<_Float16*>(base);
     float* rs = reinterpret_cast<float*>(base + rs_offset);
@@ -672,10 +703,10 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     int rc = SAMHIP_OK;
     // activation staging and weight decode in one launch (aligned rows, K <= 5120)
     bool prepared = false;
-    if (tall && aligned && K <= 5120) {
+    if (gemm16 && aligned && kp <= 5120) {
         rc = traced(ctx, prep_name(mode), w->type, M, N, K, [&]() -> int {
-            prepared = launch_prep(mode, w->type, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), M, K, a,
-                                   K, rs, x86, w->data, int64_t(w->nb[1]), N, wh, K, ctx->stream);
+            prepared = launch_prep(mode, w->type, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), M, K, kp,
+                                   a, kp, rs, x86, w->data, int64_t(w->nb[1]), N, wh, kp, ctx->stream);
             HIP_TRY(hipGetLastError(), "staging and weight decode launch");
             return prepared ? SAMHIP_OK : fail(SAMHIP_ERR_UNSUPPORTED, "mul_mat: no staging kernel for this shape");
         });
@@ -683,26 +714,26 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     }
     if (!prepared) {
         rc = traced(ctx, stage_name(mode), w->type, M, N, K, [&]() -> int {
-            launch_stage_rows(mode, aligned, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), M, K, a, K,
-                              rs, x86, ctx->stream);
+            launch_stage_rows(mode, aligned, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), M, K, kp,
+                              a, kp, rs, x86, ctx->stream);
             HIP_TRY(hipGetLastError(), "activation staging launch");
             return SAMHIP_OK;
         });
         if (rc) return rc;
     }
-    if (tall) {
+    if (gemm16) {
         if (!prepared) {
             rc = traced(ctx, dequant_name(w->type), w->type, M, N, K, [&]() -> int {
-                launch_dequant_w_f16(w->type, w->data, int64_t(w->nb[1]), N, K, wh, K, ctx->stream);
+                launch_dequant_w_f16(w->type, w->data, int64_t(w->nb[1]), N, K, kp, wh, kp, ctx->stream);
                 HIP_TRY(hipGetLastError(), "weight dequant launch");
                 return SAMHIP_OK;
             });
             if (rc) return rc;
         }
-        const int cfg = ctx->gemm_cfg >= 0 ? ctx->gemm_cfg : gemm_f16_pick_plain(M, N, K, ctx->cus);
+        const int cfg = ctx->gemm_cfg >= 0 ? ctx->gemm_cfg : gemm_f16_pick_plain(M, N, kp, ctx->cus);
         variant = gemm_f16_config_name(cfg);
         rc = traced(ctx, variant, w->type, M, N, K, [&]() -> int {
-            launch_gemm_f16(cfg, a, K, rs, wh, K, static_cast<float*>(y->data), int64_t(y->nb[1] / 4), M, N, K,
+            launch_gemm_f16(cfg, a, kp, rs, wh, kp, static_cast<float*>(y->data), int64_t(y->nb[1] / 4), M, N, kp,
                             ctx->cus, ctx->stream);
             HIP_TRY(hipGetLastError(), "gemm launch");
             return SAMHIP_OK;
@@ -729,7 +760,7 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     if (rc) return rc;
     ctx->info.mul_mat_calls++;
     ctx->info.activation_launches++;
-    if (tall || M > kSkinnyMaxM) ctx->info.gemm_launches++;
+    if (gemm16 || M > kSkinnyMaxM) ctx->info.gemm_launches++;
     ctx->info.activation_payload_peak_bytes = std::max<uint64_t>(ctx->info.activation_payload_peak_bytes, a_bytes);
     std::snprintf(ctx->info.kernel_variant, sizeof(ctx->info.kernel_variant), "%s", variant);
     return SAMHIP_OK;
@@ -944,7 +975,7 @@ int linear(samhip_context* ctx, const samhip_tensor& w, const float* x, int M, f
     int rc = traced(ctx, in ? "stage_codes_q8_0" : prep_name(mode), w.type, M, N, K, [&]() -> int {
         const bool ok = in ? launch_prep_codes(in->codes, in->amax, in->ld, M, K, a, K, rs, w.type, w.data,
                                                int64_t(w.nb[1]), N, wh, K, ctx->stream)
-                           : launch_prep(mode, w.type, x, K, M, K, a, K, rs, x86, w.data, int64_t(w.nb[1]), N, wh, K,
+                           : launch_prep(mode, w.type, x, K, M, K, K, a, K, rs, x86, w.data, int64_t(w.nb[1]), N, wh, K,
                                          ctx->stream, pre);
         if (!ok) return fail(SAMHIP_ERR_UNSUPPORTED, "%s: no staging kernel for K = %d", what, K);
         HIP_TRY(hipGetLastError(), "staging and weight decode launch");

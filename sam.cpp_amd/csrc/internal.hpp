@@ -6,7 +6,8 @@
 namespace samhip {
 
 // mode: T_F16 (direct), T_Q8_0 or T_Q8_K (native activation packing).
-void launch_stage_rows(int mode, bool aligned, const float* x, int64_t x_stride, int M, int K, _Float16* a,
+// Columns K .. kp - 1 of the operand are zeros (K a multiple of 32; lda >= kp).
+void launch_stage_rows(int mode, bool aligned, const float* x, int64_t x_stride, int M, int K, int kp, _Float16* a,
                        int64_t lda, float* row_scale, int x86, hipStream_t stream);
 
 // Q8_0 / Q8_K activation rows in ggml wire format.
@@ -35,9 +36,10 @@ void launch_quantize_weights(int type, const float* x, int64_t x_stride, int row
 void launch_dequant_rows(int type, const void* src, int64_t src_stride, const int32_t* ids, int64_t src_rows,
                          float* dst, int64_t dst_stride, int rows, int K, int* bad_id, hipStream_t stream);
 
-// Weight rows -> fp16(ggml to_float(W)) [N][K] with row stride ldo halves.
-void launch_dequant_w_f16(int wtype, const void* w, int64_t w_stride, int N, int K, _Float16* out, int64_t ldo,
-                          hipStream_t stream);
+// Weight rows -> fp16(ggml to_float(W)) [N][kp] with row stride ldo halves,
+// columns K .. kp - 1 zeros (kp a multiple of 32).
+void launch_dequant_w_f16(int wtype, const void* w, int64_t w_stride, int N, int K, int kp, _Float16* out,
+                          int64_t ldo, hipStream_t stream);
 
 // fp16 x fp16 GEMM for tall shapes: Y = rs * A B^T.  cfg < 0 picks a tile
 // configuration from the shape; returns the configuration's name.
@@ -209,8 +211,9 @@ struct RowPre {
 };
 
 // Activation staging and weight decode of a tall product in one launch
-// (16-byte aligned activation rows, K <= 5120); false when not applicable.
-bool launch_prep(int mode, int wtype, const float* x, int64_t x_stride, int M, int K, _Float16* a, int64_t lda,
+// (16-byte aligned activation rows, kp <= 5120; columns K .. kp - 1 of both
+// operands are zeros); false when not applicable.
+bool launch_prep(int mode, int wtype, const float* x, int64_t x_stride, int M, int K, int kp, _Float16* a, int64_t lda,
                  float* row_scale, int x86, const void* w, int64_t w_stride, int N, _Float16* wout, int64_t ldo,
                  hipStream_t stream, const RowPre& pre = RowPre{});
 // The same for a Q8_0 weight whose activation rows arrive as Q8_0 codes

@@ -23,7 +23,7 @@ namespace {
 // so X is read once; every cross-lane reduction runs with all lanes active
 // (lanes past K hold zeros).
 template <int MODE, int CH, bool X86, int PRE = PRE_NONE>
-__device__ __forceinline__ void stage8_row(const float* __restrict__ x, int64_t x_stride, int m, int K,
+__device__ __forceinline__ void stage8_row(const float* __restrict__ x, int64_t x_stride, int m, int K, int kp,
                                            _Float16* __restrict__ a, int64_t lda, float* __restrict__ row_scale,
                                            int lane, const RowPre& pre = RowPre{}) {
     const float* xr = x + int64_t(m) * x_stride;
@@ -111,7 +111,7 @@ __device__ __forceinline__ void stage8_row(const float* __restrict__ x, int64_t 
     for (int c = 0; c < CH; ++c) {
         const int k = 512 * c + 8 * lane;
         const half8 o = quant8<MODE, X86>(v[c], lane, down);
-        if (k < K) *reinterpret_cast<half8*>(ar + k) = o;
+        if (k < kp) *reinterpret_cast<half8*>(ar + k) = o;   // lanes in [K, kp) hold zeros
     }
 }
 
@@ -124,7 +124,7 @@ __device__ __forceinline__ void stage8_row(const float* __restrict__ x, int64_t 
 // chunked pass parking the Q8 codes in LDS until the row maximum is known:
 // 43-44 us).
 template <int MODE, bool X86, int PRE>
-__device__ __forceinline__ void stage8_half_row(const float* __restrict__ x, int64_t x_stride, int m, int M, int K,
+__device__ __forceinline__ void stage8_half_row(const float* __restrict__ x, int64_t x_stride, int m, int M, int K, int kp,
                                                 _Float16* __restrict__ a, int64_t lda, float* __restrict__ row_scale,
                                                 int lane, int wave, float* pair_max) {
     constexpr int CHH = 5;
@@ -165,27 +165,33 @@ __device__ __forceinline__ void stage8_half_row(const float* __restrict__ x, int
     for (int c = 0; c < CHH; ++c) {
         const int k = 2560 * half + 512 * c + 8 * lane;
         const half8 o = quant8<MODE, X86>(v[c], lane, down);
-        if (live && k < K) *reinterpret_cast<half8*>(ar + k) = o;
+        if (live && k < kp) *reinterpret_cast<half8*>(ar + k) = o;
     }
 }
 
 template <int MODE, int CH, bool X86>
-__global__ __launch_bounds__(256) void stage8_kernel(const float* __restrict__ x, int64_t x_stride, int M, int K,
+__global__ __launch_bounds__(256) void stage8_kernel(const float* __restrict__ x, int64_t x_stride, int M, int K, int kp,
                                                      _Float16* __restrict__ a, int64_t lda,
                                                      float* __restrict__ row_scale) {
     const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (m >= M) return;
-    stage8_row<MODE, CH, X86>(x, x_stride, m, K, a, lda, row_scale, threadIdx.x & 63);
+    stage8_row<MODE, CH, X86>(x, x_stride, m, K, kp, a, lda, row_scale, threadIdx.x & 63);
 }
 
-// thread t: half (t & 1) of 32-value step of one weight row -> 16 fp16 values
+// thread t: half (t & 1) of 32-value step of one weight row -> 16 fp16
+// values; the steps past K, up to kp, are zeros
 template <int WT>
-__device__ __forceinline__ void dequant_piece(const uint8_t* __restrict__ W, int64_t w_stride, int K, int64_t t,
-                                              _Float16* __restrict__ out, int64_t ldo) {
-    const int steps = K / 32;
+__device__ __forceinline__ void dequant_piece(const uint8_t* __restrict__ W, int64_t w_stride, int K, int kp,
+                                              int64_t t, _Float16* __restrict__ out, int64_t ldo) {
+    const int steps = kp / 32;
     const int h = int(t & 1);
     const int64_t rs = t >> 1;
     const int row = int(rs / steps), step = int(rs % steps);
+    if (32 * step >= K) {   // Q8_0 rows only: a K-quant row ends on a multiple of 256
+        half8* o = reinterpret_cast<half8*>(out + int64_t(row) * ldo + 32 * step + 16 * h);
+        o[0] = o[1] = half8{0, 0, 0, 0, 0, 0, 0, 0};
+        return;
+    }
     WeightPiece<WT> piece;
     piece.load(W + int64_t(row) * w_stride, step, h);
     _Float16 v[16];
@@ -199,7 +205,7 @@ __device__ __forceinline__ void dequant_piece(const uint8_t* __restrict__ W, int
 // [0, stage_blocks) pack four activation rows each, the rest decode 256
 // weight pieces each (the two roles touch disjoint memory).
 template <int MODE, int CH, bool X86, int WT, int PRE = PRE_NONE>
-__global__ __launch_bounds__(256) void prep_kernel(const float* __restrict__ x, int64_t x_stride, int M, int K,
+__global__ __launch_bounds__(256) void prep_kernel(const float* __restrict__ x, int64_t x_stride, int M, int K, int kp,
                                                    _Float16* __restrict__ a, int64_t lda, float* __restrict__ row_scale,
                                                    int stage_blocks, const uint8_t* __restrict__ W, int64_t w_stride,
                                                    int N, _Float16* __restrict__ wout, int64_t ldo, RowPre pre) {
@@ -209,7 +215,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const float* __restrict__ x, 
         if (int(blockIdx.x) < stage_blocks) {
             __shared__ float pair_max[4];
             const int wave = threadIdx.x >> 6;
-            stage8_half_row<MODE, X86, PRE>(x, x_stride, blockIdx.x * 2 + (wave >> 1), M, K, a, lda, row_scale,
+            stage8_half_row<MODE, X86, PRE>(x, x_stride, blockIdx.x * 2 + (wave >> 1), M, K, kp, a, lda, row_scale,
                                        threadIdx.x & 63, wave, pair_max);
             return;
         }
@@ -217,17 +223,17 @@ __global__ __launch_bounds__(256) void prep_kernel(const float* __restrict__ x, 
     if (!PAIR && int(blockIdx.x) < stage_blocks) {
         const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
         if (m < M) {
-            stage8_row<MODE, CH, X86, PRE>(x, x_stride, m, K, a, lda, row_scale, threadIdx.x & 63, pre);
+            stage8_row<MODE, CH, X86, PRE>(x, x_stride, m, K, kp, a, lda, row_scale, threadIdx.x & 63, pre);
         }
         return;
     }
     const int64_t t = int64_t(blockIdx.x - stage_blocks) * 256 + threadIdx.x;
-    if (t < int64_t(N) * (K / 32) * 2) dequant_piece<WT>(W, w_stride, K, t, wout, ldo);
+    if (t < int64_t(N) * (kp / 32) * 2) dequant_piece<WT>(W, w_stride, K, kp, t, wout, ldo);
 }
 
 // One wave per row, 4 rows per 256-thread block.
 template <int MODE>
-__global__ __launch_bounds__(256) void stage_rows_kernel(const float* __restrict__ x, int64_t x_stride, int M, int K,
+__global__ __launch_bounds__(256) void stage_rows_kernel(const float* __restrict__ x, int64_t x_stride, int M, int K, int kp,
                                                          _Float16* __restrict__ a, int64_t lda,
                                                          float* __restrict__ row_scale, int x86) {
     const int lane = threadIdx.x & 63;
@@ -264,22 +270,23 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const float* __restrict
         typedef _Float16 half4 __attribute__((ext_vector_type(4)));
         *reinterpret_cast<half4*>(ar + k) = half4{out[0], out[1], out[2], out[3]};
     }
+    for (int k = K + lane; k < kp; k += 64) ar[k] = (_Float16)0.f;
 }
 
 // Weight rows -> fp16(to_float(W)) [N][K]: thread (row, 32-element step,
 // half) writes 16 consecutive halves, so a wave stores 1 KB contiguously.
 template <int WT>
 __global__ __launch_bounds__(256) void dequant_w_f16_kernel(const uint8_t* __restrict__ W, int64_t w_stride, int N,
-                                                            int K, _Float16* __restrict__ out, int64_t ldo) {
+                                                            int K, int kp, _Float16* __restrict__ out, int64_t ldo) {
     const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (t >= int64_t(N) * (K / 32) * 2) return;
-    dequant_piece<WT>(W, w_stride, K, t, out, ldo);
+    if (t >= int64_t(N) * (kp / 32) * 2) return;
+    dequant_piece<WT>(W, w_stride, K, kp, t, out, ldo);
 }
 
 // Scalar-load variant for rows that are not 16-byte aligned.
 template <int MODE>
 __global__ __launch_bounds__(256) void stage_rows_unaligned_kernel(const float* __restrict__ x, int64_t x_stride, int M,
-                                                                   int K, _Float16* __restrict__ a, int64_t lda,
+                                                                   int K, int kp, _Float16* __restrict__ a, int64_t lda,
                                                                    float* __restrict__ row_scale, int x86) {
     const int lane = threadIdx.x & 63;
     const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -310,6 +317,7 @@ __global__ __launch_bounds__(256) void stage_rows_unaligned_kernel(const float* 
         for (int i = 0; i < 4; ++i)
             ar[k + i] = MODE == T_F16 ? (_Float16)(v[i] * down) : (_Float16)((float)q[i] * dd);
     }
+    for (int k = K + lane; k < kp; k += 64) ar[k] = (_Float16)0.f;
 }
 
 // Q8_0 / Q8_K rows in ggml wire format.  One wave per row.
@@ -463,33 +471,33 @@ __global__ __launch_bounds__(256) void prep_codes_kernel(const int8_t* __restric
         return;
     }
     const int64_t t = int64_t(blockIdx.x - stage_blocks) * 256 + threadIdx.x;
-    if (t < int64_t(N) * (K / 32) * 2) dequant_piece<WT>(W, w_stride, K, t, wout, ldo);
+    if (t < int64_t(N) * (K / 32) * 2) dequant_piece<WT>(W, w_stride, K, K, t, wout, ldo);
 }
 
 }  // namespace
 
-void launch_dequant_w_f16(int wtype, const void* w, int64_t w_stride, int N, int K, _Float16* out, int64_t ldo,
-                          hipStream_t stream) {
-    const int64_t threads = int64_t(N) * (K / 32) * 2;
+void launch_dequant_w_f16(int wtype, const void* w, int64_t w_stride, int N, int K, int kp, _Float16* out,
+                          int64_t ldo, hipStream_t stream) {
+    const int64_t threads = int64_t(N) * (kp / 32) * 2;
     const dim3 grid(unsigned((threads + 255) / 256)), block(256);
     const uint8_t* wb = static_cast<const uint8_t*>(w);
     switch (wtype) {
-        case T_Q8_0: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q8_0>, grid, block, 0, stream, wb, w_stride, N, K, out, ldo); break;
-        case T_Q4_K: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q4_K>, grid, block, 0, stream, wb, w_stride, N, K, out, ldo); break;
-        case T_Q5_K: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q5_K>, grid, block, 0, stream, wb, w_stride, N, K, out, ldo); break;
-        case T_Q6_K: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q6_K>, grid, block, 0, stream, wb, w_stride, N, K, out, ldo); break;
+        case T_Q8_0: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q8_0>, grid, block, 0, stream, wb, w_stride, N, K, kp, out, ldo); break;
+        case T_Q4_K: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q4_K>, grid, block, 0, stream, wb, w_stride, N, K, kp, out, ldo); break;
+        case T_Q5_K: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q5_K>, grid, block, 0, stream, wb, w_stride, N, K, kp, out, ldo); break;
+        case T_Q6_K: hipLaunchKernelGGL(dequant_w_f16_kernel<T_Q6_K>, grid, block, 0, stream, wb, w_stride, N, K, kp, out, ldo); break;
         default: break;
     }
 }
 
-bool launch_prep(int mode, int wtype, const float* x, int64_t x_stride, int M, int K, _Float16* a, int64_t lda,
+bool launch_prep(int mode, int wtype, const float* x, int64_t x_stride, int M, int K, int kp, _Float16* a, int64_t lda,
                  float* row_scale, int x86, const void* w, int64_t w_stride, int N, _Float16* wout, int64_t ldo,
                  hipStream_t stream, const RowPre& pre) {
-    if (K > 512 * 10 || reinterpret_cast<uintptr_t>(x) % 16 || x_stride % 4) return false;
+    if (kp > 512 * 10 || reinterpret_cast<uintptr_t>(x) % 16 || x_stride % 4) return false;
     if (pre.kind == PRE_LAYER_NORM && (!pre.w || !pre.b || reinterpret_cast<uintptr_t>(pre.w) % 16 ||
                                        reinterpret_cast<uintptr_t>(pre.b) % 16 || K % 8))
         return false;
-    const int64_t db = (int64_t(N) * (K / 32) * 2 + 255) / 256;
+    const int64_t db = (int64_t(N) * (kp / 32) * 2 + 255) / 256;
     const dim3 block(256);
     const uint8_t* wb = static_cast<const uint8_t*>(w);
 #define SAMHIP_PREP(MODE, CH, X86, WT)                                                                               \
@@ -499,18 +507,18 @@ bool launch_prep(int mode, int wtype, const float* x, int64_t x_stride, int M, i
         const dim3 grid(unsigned(sb + db));                                                                          \
         if (pre.kind == PRE_GELU)                                                                                    \
             hipLaunchKernelGGL((prep_kernel<MODE, CH, X86, WT, PRE_GELU>), grid, block, 0, stream, x, x_stride, M, K, \
-                               a, lda, row_scale, sb, wb, w_stride, N, wout, ldo, pre);                              \
+                               kp, a, lda, row_scale, sb, wb, w_stride, N, wout, ldo, pre);                              \
         else if (pre.kind == PRE_LAYER_NORM)                                                                         \
             hipLaunchKernelGGL((prep_kernel<MODE, CH, X86, WT, PRE_LAYER_NORM>), grid, block, 0, stream, x, x_stride, \
-                               M, K, a, lda, row_scale, sb, wb, w_stride, N, wout, ldo, pre);                        \
+                               M, K, kp, a, lda, row_scale, sb, wb, w_stride, N, wout, ldo, pre);                        \
         else                                                                                                         \
-            hipLaunchKernelGGL((prep_kernel<MODE, CH, X86, WT>), grid, block, 0, stream, x, x_stride, M, K, a, lda,  \
+            hipLaunchKernelGGL((prep_kernel<MODE, CH, X86, WT>), grid, block, 0, stream, x, x_stride, M, K, kp, a, lda,  \
                                row_scale, sb, wb, w_stride, N, wout, ldo, pre);                                      \
     } while (0)
 #define SAMHIP_PREP_CH(MODE, X86, WT)                    \
     do {                                                 \
-        if (K <= 1024) SAMHIP_PREP(MODE, 2, X86, WT);    \
-        else if (K <= 2048) SAMHIP_PREP(MODE, 4, X86, WT); \
+        if (kp <= 1024) SAMHIP_PREP(MODE, 2, X86, WT);    \
+        else if (kp <= 2048) SAMHIP_PREP(MODE, 4, X86, WT); \
         else SAMHIP_PREP(MODE, 10, X86, WT);             \
     } while (0)
     switch (wtype) {
@@ -553,22 +561,22 @@ bool launch_prep_codes(const int8_t* codes, const float* amax, int64_t ldc, int 
     return true;
 }
 
-void launch_stage_rows(int mode, bool aligned, const float* x, int64_t x_stride, int M, int K, _Float16* a,
+void launch_stage_rows(int mode, bool aligned, const float* x, int64_t x_stride, int M, int K, int kp, _Float16* a,
                        int64_t lda, float* row_scale, int x86, hipStream_t stream) {
     const dim3 grid((M + 3) / 4), block(256);
-    if (aligned && K <= 512 * 10) {
+    if (aligned && kp <= 512 * 10) {
 #define SAMHIP_STAGE8(MODE, CH)                                                                                 \
     do {                                                                                                        \
         if (MODE == T_Q8_0 && x86)                                                                              \
-            hipLaunchKernelGGL((stage8_kernel<MODE, CH, true>), grid, block, 0, stream, x, x_stride, M, K, a,   \
+            hipLaunchKernelGGL((stage8_kernel<MODE, CH, true>), grid, block, 0, stream, x, x_stride, M, K, kp, a, \
                                lda, row_scale);                                                                 \
         else                                                                                                    \
-            hipLaunchKernelGGL((stage8_kernel<MODE, CH, false>), grid, block, 0, stream, x, x_stride, M, K, a,  \
+            hipLaunchKernelGGL((stage8_kernel<MODE, CH, false>), grid, block, 0, stream, x, x_stride, M, K, kp, a, \
                                lda, row_scale);                                                                 \
     } while (0)
 #define SAMHIP_STAGE8_MODE(MODE)                  \
-    if (K <= 1024) SAMHIP_STAGE8(MODE, 2);        \
-    else if (K <= 2048) SAMHIP_STAGE8(MODE, 4);   \
+    if (kp <= 1024) SAMHIP_STAGE8(MODE, 2);       \
+    else if (kp <= 2048) SAMHIP_STAGE8(MODE, 4);   \
     else SAMHIP_STAGE8(MODE, 10);
         switch (mode) {
             case T_F16: SAMHIP_STAGE8_MODE(T_F16) break;
@@ -581,9 +589,9 @@ void launch_stage_rows(int mode, bool aligned, const float* x, int64_t x_stride,
         return;
     }
 #define SAMHIP_STAGE(MODE)                                                                                      \
-    if (aligned) hipLaunchKernelGGL(stage_rows_kernel<MODE>, grid, block, 0, stream, x, x_stride, M, K, a, lda, \
+    if (aligned) hipLaunchKernelGGL(stage_rows_kernel<MODE>, grid, block, 0, stream, x, x_stride, M, K, kp, a, lda, \
                                     row_scale, x86);                                                           \
-    else hipLaunchKernelGGL(stage_rows_unaligned_kernel<MODE>, grid, block, 0, stream, x, x_stride, M, K, a, lda, \
+    else hipLaunchKernelGGL(stage_rows_unaligned_kernel<MODE>, grid, block, 0, stream, x, x_stride, M, K, kp, a, lda, \
                             row_scale, x86);
     switch (mode) {
         case T_F16: SAMHIP_STAGE(T_F16) break;
