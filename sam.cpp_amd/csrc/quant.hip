@@ -322,41 +322,78 @@ __global__ __launch_bounds__(256) void stage_rows_unaligned_kernel(const float* 
     for (int k = K + lane; k < kp; k += 64) ar[k] = (_Float16)0.f;
 }
 
-// Q8_0 / Q8_K rows in ggml wire format.  One wave per row.
-template <int TYPE>
-__global__ __launch_bounds__(256) void quantize_act_kernel(const float* __restrict__ x, int64_t x_stride, int rows,
-                                                           int K, uint8_t* __restrict__ dst, int x86) {
+// Q8_K rows in ggml wire format.  One wave per row.
+__global__ __launch_bounds__(256) void quantize_q8_k_kernel(const float* __restrict__ x, int64_t x_stride, int rows,
+                                                            int K, uint8_t* __restrict__ dst) {
     const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= rows) return;
     const float* xr = x + int64_t(r) * x_stride;
-    constexpr int BE = block_elems(TYPE), BB = block_bytes(TYPE);
-    uint8_t* out = dst + int64_t(r) * (K / BE) * BB;
+    uint8_t* out = dst + int64_t(r) * (K / 256) * 292;
     for (int k = 4 * lane; k < K; k += 256) {
         const floatx4 v = floatx4{xr[k], xr[k + 1], xr[k + 2], xr[k + 3]};
         float d;
         int q[4];
-        if (TYPE == T_Q8_0) q8_0_codes(v, x86, d, q);
-        else q8_k_codes(v, lane, d, q);
-        uint8_t* blk = out + (k / BE) * BB;
-        const int within = k % BE;
-        if (TYPE == T_Q8_0) {
-            if (within == 0) {
-                const uint16_t h = float_to_half_bits(d);
-                blk[0] = uint8_t(h & 0xff);
-                blk[1] = uint8_t(h >> 8);
-            }
-            for (int i = 0; i < 4; ++i) blk[2 + within + i] = uint8_t(int8_t(q[i]));
-        } else {
-            if (within == 0) *reinterpret_cast<float*>(blk) = d;
-            for (int i = 0; i < 4; ++i) blk[4 + within + i] = uint8_t(int8_t(q[i]));
-            const int s = group_sum<4>(q[0] + q[1] + q[2] + q[3]);
-            if ((lane & 3) == 0) {
-                const int16_t s16 = int16_t(s);
-                blk[260 + 2 * (within / 16)] = uint8_t(uint16_t(s16) & 0xff);
-                blk[260 + 2 * (within / 16) + 1] = uint8_t(uint16_t(s16) >> 8);
-            }
+        q8_k_codes(v, lane, d, q);
+        uint8_t* blk = out + (k / 256) * 292;
+        const int within = k % 256;
+        if (within == 0) *reinterpret_cast<float*>(blk) = d;
+        for (int i = 0; i < 4; ++i) blk[4 + within + i] = uint8_t(int8_t(q[i]));
+        const int s = group_sum<4>(q[0] + q[1] + q[2] + q[3]);
+        if ((lane & 3) == 0) {
+            const int16_t s16 = int16_t(s);
+            blk[260 + 2 * (within / 16)] = uint8_t(uint16_t(s16) & 0xff);
+            blk[260 + 2 * (within / 16) + 1] = uint8_t(uint16_t(s16) >> 8);
         }
+    }
+}
+
+// Q8_0 rows in ggml wire format.  Packed rows follow one another without
+// padding, so the kernel walks the blocks of all rows as one sequence: a wave
+// takes 16 of them (8 values a lane, a block on a lane quad), puts their 544
+// bytes together in LDS and stores them as dwords.  (With a wave per row and
+// a store per code byte, the 34-byte blocks cost five stores a lane and 256
+// values.)  Bound by HBM: 82 944 rows of 256 values 20.7 -> 16.8 us.
+constexpr int kQ8WaveBlocks = 16, kQ8WaveBytes = 34 * kQ8WaveBlocks;
+
+template <bool X86, bool XVEC>
+__global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restrict__ x, int64_t x_stride,
+                                                            int64_t blocks, int nb, uint8_t* __restrict__ dst) {
+    __shared__ __attribute__((aligned(16))) uint8_t buf[4][kQ8WaveBytes];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t first = (int64_t(blockIdx.x) * 4 + wave) * kQ8WaveBlocks;
+    if (first >= blocks) return;   // (no barrier below: a wave's bytes are its own)
+    const int i = lane >> 2;
+    // lanes past the last block repeat it; their bytes are not stored
+    const int64_t g = min(first + i, blocks - 1);
+    const int64_t r = blocks <= 0xffffffff ? int64_t(uint32_t(g) / uint32_t(nb)) : g / nb;
+    const float* xb = x + r * x_stride + 32 * (g - r * nb) + 8 * (lane & 3);
+    floatx8 v;
+    if (XVEC) {
+        const floatx4 a = load4f(xb), c = load4f(xb + 4);
+        v = floatx8{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = xb[j];
+    }
+    float d;
+    int q[8];
+    quant8_icodes<T_Q8_0, X86>(v, lane, d, q);
+    uint16_t* o = reinterpret_cast<uint16_t*>(buf[wave] + 34 * i);
+    if ((lane & 3) == 0) o[0] = float_to_half_bits(d);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[1 + 4 * (lane & 3) + j] = uint16_t((q[2 * j] & 0xff) | ((q[2 * j + 1] & 0xff) << 8));
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the wave's bytes are in LDS
+    __builtin_amdgcn_wave_barrier();
+    const int bytes = int(min(int64_t(kQ8WaveBlocks), blocks - first)) * 34;
+    uint8_t* out = dst + first * 34;
+    if (reinterpret_cast<uintptr_t>(dst) % 4 == 0) {
+        for (int k = 4 * lane; k + 4 <= bytes; k += 256)
+            *reinterpret_cast<uint32_t*>(out + k) = *reinterpret_cast<const uint32_t*>(buf[wave] + k);
+        const int left = bytes & 3, at = bytes - left;
+        if (lane < left) out[at + lane] = buf[wave][at + lane];
+    } else {
+        for (int k = lane; k < bytes; k += 64) out[k] = buf[wave][k];
     }
 }
 
@@ -629,13 +666,22 @@ void launch_cast_f16(const float* x, int64_t x_stride, int rows, int K, _Float16
 
 void launch_quantize_act(int type, const float* x, int64_t x_stride, int rows, int K, void* dst, int x86,
                          hipStream_t stream) {
-    const dim3 grid((rows + 3) / 4), block(256);
-    if (type == T_Q8_0)
-        hipLaunchKernelGGL(quantize_act_kernel<T_Q8_0>, grid, block, 0, stream, x, x_stride, rows, K,
-                           static_cast<uint8_t*>(dst), x86);
-    else
-        hipLaunchKernelGGL(quantize_act_kernel<T_Q8_K>, grid, block, 0, stream, x, x_stride, rows, K,
-                           static_cast<uint8_t*>(dst), x86);
+    uint8_t* d = static_cast<uint8_t*>(dst);
+    if (type != T_Q8_0) {
+        hipLaunchKernelGGL(quantize_q8_k_kernel, dim3((rows + 3) / 4), dim3(256), 0, stream, x, x_stride, rows, K, d);
+        return;
+    }
+    const int nb = K / 32;
+    const int64_t blocks = int64_t(rows) * nb;
+    const dim3 grid(unsigned((blocks + 4 * kQ8WaveBlocks - 1) / (4 * kQ8WaveBlocks)));
+    const bool xvec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && x_stride % 4 == 0;
+#define SAMHIP_Q8_0(X86, XVEC) \
+    hipLaunchKernelGGL((quantize_q8_0_kernel<X86, XVEC>), grid, dim3(256), 0, stream, x, x_stride, blocks, nb, d)
+    if (x86 && xvec) SAMHIP_Q8_0(true, true);
+    else if (x86) SAMHIP_Q8_0(true, false);
+    else if (xvec) SAMHIP_Q8_0(false, true);
+    else SAMHIP_Q8_0(false, false);
+#undef SAMHIP_Q8_0
 }
 
 // ---------------------------------------------------------------------------
