@@ -376,9 +376,18 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restr
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = xb[j];
     }
-    float d;
+    // as quant8_icodes, except that a block of NaNs keeps a NaN scale
+    float amax = fabsf(v[0]);
+#pragma unroll
+    for (int j = 1; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+    amax = max4_lanes(amax);
+    const float d = div127(amax);
+    float mul;
+    if (X86) mul = amax != 0.f ? 127.f / amax : 0.f;
+    else mul = d != 0.f ? 1.f / d : 0.f;
     int q[8];
-    quant8_icodes<T_Q8_0, X86>(v, lane, d, q);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) q[j] = cvt_i32_nan0(quant8_round<T_Q8_0, X86>(v[j] * mul));
     uint16_t* o = reinterpret_cast<uint16_t*>(buf[wave] + 34 * i);
     if ((lane & 3) == 0) o[0] = float_to_half_bits(d);
 #pragma unroll

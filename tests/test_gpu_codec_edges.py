@@ -69,3 +69,16 @@ def test_quantize_q8_0_edges(gpu_ctx, oracle, samhip, rounding, rows, k, src_off
     assert (got[:dst_off] == 0xA5).all() and (got[dst_off + ref.size:] == 0xA5).all()
     sbuf.free()
     dbuf.free()
+
+
+@pytest.mark.parametrize("rounding", ["x86", "ref"])
+def test_quantize_q8_0_nan_blocks(gpu_ctx, samhip, rounding):
+    """NaN packs as code 0; a block of nothing else keeps a NaN scale, one with a finite value that value's."""
+    x = np.full((3, 64), np.nan, np.float32)
+    x[1, 5] = -127.0
+    x[2] = 1.0
+    got = gpu_ctx.quantize(8, x, samhip.ROUND_X86 if rounding == "x86" else samhip.ROUND_REF).reshape(3, 2, 34)
+    scale = np.ascontiguousarray(got[:, :, :2]).view(np.float16)[:, :, 0]
+    assert np.isnan(scale[0]).all() and scale[1, 0] == 1.0 and np.isnan(scale[1, 1])
+    codes = got[:, :, 2:].view(np.int8)
+    assert (codes[0] == 0).all() and codes[1, 0, 5] == -127 and np.count_nonzero(codes[1]) == 1 and (codes[2] == 127).all()
