@@ -68,12 +68,6 @@ __device__ __forceinline__ float group_max(float v) {
     return v;
 }
 
-template <int width>
-__device__ __forceinline__ int group_sum(int v) {
-    for (int off = width / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // 2^e as a float for |e| <= 126.
 __device__ __forceinline__ float exp2i(int e) { return __builtin_bit_cast(float, uint32_t(127 + e) << 23); }
 
@@ -109,11 +103,21 @@ __device__ __forceinline__ floatx4 load4f_stream(const float* p) {
 // for lane ^ 1 and lane ^ 2, row rotations by 4 and 8 within 16 lanes.
 constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;
 
+// (bound_ctrl: every lane these patterns read exists, and with it the
+// compiler folds the move into the instruction that uses it)
 template <int CTRL>
-__device__ __forceinline__ int dpp(int v) { return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, false); }
+__device__ __forceinline__ int dpp(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+    return __builtin_bit_cast(float, dpp<CTRL>(__builtin_bit_cast(int, v)));
+}
+
+// sum over aligned groups of 2 or 4 lanes
+template <int width>
+__device__ __forceinline__ int group_sum(int v) {
+    static_assert(width == 2 || width == 4, "a lane pair or quad");
+    v += dpp<DPP_XOR1>(v);
+    return width == 4 ? v + dpp<DPP_XOR2>(v) : v;
 }
 
 __device__ __forceinline__ float max4_lanes(float v) {
@@ -132,6 +136,28 @@ __device__ __forceinline__ int min32_lanes(int v) {
     v = min(v, dpp<DPP_ROR4>(v));
     v = min(v, dpp<DPP_ROR8>(v));
     return min(v, __shfl_xor(v, 16, 64));
+}
+
+// Maxima of magnitudes as the unsigned integers of their bits: the order is
+// the floats' own, a NaN sorts above infinity, and the steps need no float
+// canonicalization.  xor16 and xor32 swap rows between two registers
+// (v_permlane16_swap, v_permlane32_swap) instead of going through LDS.
+constexpr uint32_t INF_BITS = 0x7f800000u;
+constexpr uint32_t TINY_BITS = 0x0d800000u;   // 2^-100: 127 / x and 1 / (x / 127) are finite from here on
+__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+template <int CTRL>
+__device__ __forceinline__ uint32_t umax_dpp(uint32_t v) { return umax(v, uint32_t(dpp<CTRL>(int(v)))); }
+__device__ __forceinline__ uint32_t umax_quad(uint32_t v) { return umax_dpp<DPP_XOR2>(umax_dpp<DPP_XOR1>(v)); }
+__device__ __forceinline__ uint32_t umax_row(uint32_t v) {   // from quads to the 16 lanes
+    return umax_dpp<DPP_ROR8>(umax_dpp<DPP_ROR4>(v));
+}
+__device__ __forceinline__ uint32_t umax_xor16(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return umax(r[0], r[1]);
+}
+__device__ __forceinline__ uint32_t umax_xor32(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return umax(r[0], r[1]);
 }
 typedef float floatx8 __attribute__((ext_vector_type(8)));
 
@@ -152,28 +178,93 @@ __device__ __forceinline__ float div127(float x) {
 // The Q8 block packing of 8 consecutive activations held by each lane;
 // lanes 4g..4g+3 hold one Q8_0 block, lanes 32h..32h+31 one Q8_K block.
 // Every lane of the wave must call these (cross-lane reductions); lanes past
-// the row's end hold zeros.  quant8_scale gives the block's decoded scale d
-// (the stored fp16 for Q8_0) and the multiplier that takes a value to its
-// unrounded code; quant8_codes and quant8_icodes give the codes in
-// [-127, 127] as floats or as ints.  X86 selects the Q8_0 rounding of
-// ggml's x86-64 from_float (scale 127/amax, ties to even) over the reference
+// the row's end hold zeros.  X86 selects the Q8_0 rounding of ggml's x86-64
+// from_float (scale 127/amax, ties to even) over the reference
 // quantize_row_q8_0_ref (scale 1/d, ties away from zero).
+//
+// quant8_extreme gives the block's extreme as float bits: its largest
+// magnitude, for Q8_K with the sign of the first element that has it (in
+// F16 mode the lane's own largest magnitude).  `odd` is set on lanes of a
+// block that holds a NaN or an infinity or whose scale may overflow, and, for
+// Q8_K, of one whose largest positive and negative values tie, where the
+// order of the elements decides: the caller then takes quant8_scale_ordered for the whole wave.  (Carrying
+// every element's index through the reduction took ~60 of the ~190 VALU
+// instructions of 8 values and two LDS round trips: text stream Q4_K, M = 32,
+// 97 products 925 -> 883 us; fusion layers Q6_K 637 -> 609; a 5184 x 1024 x
+// 3072 Q4_K product 52.0 -> 51.3.)
+template <int MODE>
+__device__ __forceinline__ uint32_t quant8_extreme(const floatx8& v, bool& odd) {
+    if (MODE == T_Q8_K) {
+        // IEEE maxima: a NaN anywhere gives NaN
+        float p = 0.f, m = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+            p = __builtin_elementwise_maximum(p, __builtin_elementwise_maximum(v[i], v[i + 1]));
+            m = __builtin_elementwise_maximum(m, __builtin_elementwise_maximum(-v[i], -v[i + 1]));
+        }
+        uint32_t pos = umax_row(umax_quad(__float_as_uint(p)));
+        uint32_t neg = umax_row(umax_quad(__float_as_uint(m)));
+        // rows [p0 n0 p2 n2] and [p1 n1 p3 n3], then both maxima on both rows
+        const auto r = __builtin_amdgcn_permlane16_swap(pos, neg, false, false);
+        const uint32_t both = umax(r[0], r[1]);
+        const auto t = __builtin_amdgcn_permlane16_swap(both, both, false, false);
+        pos = t[0];
+        neg = t[1];
+        const uint32_t amax = umax(pos, neg);
+        odd = odd || (amax != 0 && (amax - TINY_BITS >= INF_BITS - TINY_BITS || pos == neg));
+        return neg > pos ? amax | 0x80000000u : amax;
+    }
+    float a = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2)
+        a = __builtin_elementwise_maximum(a, __builtin_elementwise_maximum(fabsf(v[i]), fabsf(v[i + 1])));
+    uint32_t amax = __float_as_uint(a) & 0x7fffffffu;   // (a NaN may carry a sign)
+    if (MODE == T_Q8_0) amax = umax_quad(amax);
+    odd = odd || (amax != 0 && amax - (MODE == T_F16 ? 0 : TINY_BITS) >= INF_BITS - (MODE == T_F16 ? 0 : TINY_BITS));
+    return amax;
+}
+
+// The largest magnitude over the wave's 64 lanes from the blocks' extremes.
+template <int MODE>
+__device__ __forceinline__ float quant8_wave_max(uint32_t extreme) {
+    uint32_t m = extreme & 0x7fffffffu;
+    if (MODE == T_F16) m = umax_quad(m);
+    if (MODE != T_Q8_K) m = umax_xor16(umax_row(m));
+    return __uint_as_float(umax_xor32(m));
+}
+
+// The block's decoded scale d (the stored fp16 for Q8_0) and the multiplier
+// that takes a value to its unrounded code, from its (finite) extreme.
 template <int MODE, bool X86>
-__device__ __forceinline__ void quant8_scale(const floatx8& v, int lane, float& d, float& mul) {
+__device__ __forceinline__ void quant8_scale_of(uint32_t extreme, float& d, float& mul) {
 #pragma clang fp contract(off)
-    d = 0.f;
-    mul = 0.f;
+    const float e = __uint_as_float(extreme);
+    if (MODE == T_Q8_0) {
+        const float dd = div127(e);
+        if (X86) mul = e != 0.f ? 127.f / e : 0.f;
+        else mul = dd != 0.f ? 1.f / dd : 0.f;
+        d = half_bits_to_float(float_to_half_bits(dd));   // stored fp16 scale
+    } else {
+        // ggml clamps the code to 127; with |v| <= |e| the product is at most
+        // 127 (1 + 2^-23), which rounds to 127, so the clamp never acts (a
+        // non-finite maximum makes the product NaN)
+        mul = -127.f / e;
+        d = 1.f / mul;
+        if (e == 0.f) mul = d = 0.f;
+    }
+}
+
+// The same from the values themselves, in element order (Q8_K: the first
+// element of largest magnitude), NaNs ignored.
+template <int MODE, bool X86>
+__device__ __forceinline__ void quant8_scale_ordered(const floatx8& v, int lane, float& d, float& mul) {
+#pragma clang fp contract(off)
     if (MODE == T_Q8_0) {
         float amax = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-        amax = max4_lanes(amax);
-        const float dd = div127(amax);
-        if (X86) mul = amax != 0.f ? 127.f / amax : 0.f;
-        else mul = dd != 0.f ? 1.f / dd : 0.f;
-        d = half_bits_to_float(float_to_half_bits(dd));   // stored fp16 scale
+        quant8_scale_of<MODE, X86>(umax_quad(__float_as_uint(amax)), d, mul);
     } else {
-        // Q8_K: first element of largest magnitude in the 256-value block
         const int base = 8 * (lane & 31);
         float la = 0.f, ls = 0.f;
         int li = 1 << 20;
@@ -186,15 +277,19 @@ __device__ __forceinline__ void quant8_scale(const floatx8& v, int lane, float& 
         // the first maximum is +-amax), so no lane-to-lane read is needed
         const float amax = max32_lanes(la);
         const int key = min32_lanes(la == amax ? 2 * li + int(__float_as_uint(ls) >> 31) : (1 << 20));
-        const float smax = (key & 1) ? -amax : amax;
-        if (amax != 0.f) {
-            // ggml clamps the code to 127; with |v| <= amax = |smax| the
-            // product is at most 127 (1 + 2^-23), which rounds to 127, so
-            // the clamp never acts (a non-finite amax makes the product NaN)
-            mul = -127.f / smax;
-            d = 1.f / mul;
-        }
+        quant8_scale_of<MODE, X86>(__float_as_uint((key & 1) ? -amax : amax), d, mul);
     }
+}
+
+// Either, for one group of blocks; true when a value of the wave may be NaN.
+template <int MODE, bool X86>
+__device__ __forceinline__ bool quant8_scale(const floatx8& v, int lane, float& d, float& mul) {
+    bool odd = false;
+    const uint32_t e = quant8_extreme<MODE>(v, odd);
+    const bool any = __any(odd);
+    if (any) quant8_scale_ordered<MODE, X86>(v, lane, d, mul);
+    else quant8_scale_of<MODE, X86>(e, d, mul);
+    return any;
 }
 
 // The rounding of a scaled value to its code.
@@ -203,25 +298,14 @@ __device__ __forceinline__ float quant8_round(float s) {
     return (MODE == T_Q8_0 && !X86) ? __builtin_roundf(s) : __builtin_rintf(s);
 }
 
-template <int MODE, bool X86>
-__device__ __forceinline__ void quant8_codes(const floatx8& v, int lane, float& d, float (&q)[8]) {
-#pragma clang fp contract(off)
-    float mul;
-    quant8_scale<MODE, X86>(v, lane, d, mul);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float r = quant8_round<MODE, X86>(v[i] * mul);
-        q[i] = r == r ? r : 0.f;   // a NaN activation packs as code 0 (this library's contract, above)
-    }
-}
-
-// The same codes as integers (the int8 kernels): the conversion itself
-// takes a NaN to 0.
+// The codes in [-127, 127] as integers (the int8 kernels): the conversion
+// itself takes a NaN to 0.
 template <int MODE, bool X86>
 __device__ __forceinline__ void quant8_icodes(const floatx8& v, int lane, float& d, int (&c)[8]) {
 #pragma clang fp contract(off)
     float mul;
-    quant8_scale<MODE, X86>(v, lane, d, mul);
+    if (MODE == T_Q8_0) quant8_scale_ordered<MODE, X86>(v, lane, d, mul);   // a quad's maximum: no order to keep
+    else quant8_scale<MODE, X86>(v, lane, d, mul);
 #pragma unroll
     for (int i = 0; i < 8; ++i) c[i] = cvt_i32_nan0(quant8_round<MODE, X86>(v[i] * mul));
 }
@@ -232,9 +316,10 @@ __device__ __forceinline__ void quant8_icodes(const floatx8& v, int lane, float&
 // q * (d * down) is fl(d * q) * down whenever d * q is a normal float (a
 // subnormal d * q is below 2^-126, and such a value times down is below
 // fp16's range unless the row maximum is below ~2^-87, where this form
-// keeps more bits).
-template <int MODE, bool X86>
-__device__ __forceinline__ half8 quant8(const floatx8& v, int lane, float down) {
+// keeps more bits).  NAN0: a NaN activation packs as code 0 (this library's
+// contract, above).
+template <int MODE, bool X86, bool NAN0>
+__device__ __forceinline__ half8 quant8_operand(const floatx8& v, float d, float mul, float down) {
 #pragma clang fp contract(off)
     half8 o;
     if (MODE == T_F16) {
@@ -242,12 +327,22 @@ __device__ __forceinline__ half8 quant8(const floatx8& v, int lane, float down) 
         for (int i = 0; i < 8; ++i) o[i] = (_Float16)(v[i] * down);
         return o;
     }
-    float d, q[8];
-    quant8_codes<MODE, X86>(v, lane, d, q);
     const float dd = d * down;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = (_Float16)(q[i] * dd);
+    for (int i = 0; i < 8; ++i) {
+        float q = quant8_round<MODE, X86>(v[i] * mul);
+        if (NAN0) q = q == q ? q : 0.f;
+        o[i] = (_Float16)(q * dd);
+    }
     return o;
+}
+
+template <int MODE, bool X86>
+__device__ __forceinline__ half8 quant8(const floatx8& v, int lane, float down) {
+    float d = 0.f, mul = 0.f;
+    bool any = false;
+    if (MODE != T_F16) any = quant8_scale<MODE, X86>(v, lane, d, mul);
+    return any ? quant8_operand<MODE, X86, true>(v, d, mul, down) : quant8_operand<MODE, X86, false>(v, d, mul, down);
 }
 
 // Q8_0 block: amax over 8 lanes x 4 values; returns fp16 d bits and codes.

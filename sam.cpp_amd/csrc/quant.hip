@@ -98,6 +98,31 @@ __device__ __forceinline__ void stage8_row(const float* __restrict__ x, int64_t 
             dst = int64_t(win) * pre.ws * pre.ws + (gy % pre.ws) * pre.ws + gx % pre.ws;
         }
     }
+    // the blocks' extremes give the row's largest magnitude and, unless a
+    // NaN, an infinity or a tie of signs sends the wave the ordered way, the
+    // blocks' scales
+    uint32_t ext[CH], top = 0;
+    bool odd = false;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        ext[c] = quant8_extreme<MODE>(v[c], odd);
+        top = umax(top, ext[c] & 0x7fffffffu);
+    }
+    _Float16* ar = a + dst * lda;
+    if (!__any(odd)) {
+        const int e = row_exponent(quant8_wave_max<MODE>(top));
+        const float down = exp2i(-e);
+        if (lane == 0) row_scale[dst] = exp2i(e);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int k = 512 * c + 8 * lane;
+            float d = 0.f, mul = 0.f;
+            if (MODE != T_F16) quant8_scale_of<MODE, X86>(ext[c], d, mul);
+            const half8 o = quant8_operand<MODE, X86, false>(v[c], d, mul, down);
+            if (k < kp) *reinterpret_cast<half8*>(ar + k) = o;   // lanes in [K, kp) hold zeros
+        }
+        return;
+    }
     float rmax = 0.f;
 #pragma unroll
     for (int c = 0; c < CH; ++c)
@@ -108,12 +133,13 @@ __device__ __forceinline__ void stage8_row(const float* __restrict__ x, int64_t 
     const int e = row_exponent(rmax);
     const float down = exp2i(-e);
     if (lane == 0) row_scale[dst] = exp2i(e);
-    _Float16* ar = a + dst * lda;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
         const int k = 512 * c + 8 * lane;
-        const half8 o = quant8<MODE, X86>(v[c], lane, down);
-        if (k < kp) *reinterpret_cast<half8*>(ar + k) = o;   // lanes in [K, kp) hold zeros
+        float d = 0.f, mul = 0.f;
+        if (MODE != T_F16) quant8_scale_ordered<MODE, X86>(v[c], lane, d, mul);
+        const half8 o = quant8_operand<MODE, X86, true>(v[c], d, mul, down);
+        if (k < kp) *reinterpret_cast<half8*>(ar + k) = o;
     }
 }
 
@@ -149,13 +175,25 @@ __device__ __forceinline__ void stage8_half_row(const float* __restrict__ x, int
         for (int c = 0; c < CHH; ++c)
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[c][i] = gelu_erf(v[c][i]);   // gelu(0) = 0 keeps the padding
-    float rmax = 0.f;
+    // as in stage8_row; the two halves meet on the largest magnitude
+    uint32_t ext[CHH], top = 0;
+    bool odd = false;
 #pragma unroll
-    for (int c = 0; c < CHH; ++c)
+    for (int c = 0; c < CHH; ++c) {
+        ext[c] = quant8_extreme<MODE>(v[c], odd);
+        top = umax(top, ext[c] & 0x7fffffffu);
+    }
+    float rmax = quant8_wave_max<MODE>(top);
+    odd = __any(odd);
+    if (odd) {   // the largest magnitude without the NaNs
+        rmax = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) rmax = fmaxf(rmax, fabsf(v[c][i]));
-    const float r32 = max32_lanes(rmax);
-    rmax = fmaxf(r32, __shfl_xor(r32, 32, 64));
+        for (int c = 0; c < CHH; ++c)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) rmax = fmaxf(rmax, fabsf(v[c][i]));
+        const float r32 = max32_lanes(rmax);
+        rmax = fmaxf(r32, __shfl_xor(r32, 32, 64));
+    }
     if (lane == 0) pair_max[wave] = rmax;
     __syncthreads();
     rmax = fmaxf(pair_max[wave & ~1], pair_max[wave | 1]);
@@ -163,10 +201,23 @@ __device__ __forceinline__ void stage8_half_row(const float* __restrict__ x, int
     const float down = exp2i(-e);
     if (live && half == 0 && lane == 0) row_scale[m] = exp2i(e);
     _Float16* ar = a + int64_t(live ? m : 0) * lda;
+    if (odd) {
+#pragma unroll
+        for (int c = 0; c < CHH; ++c) {
+            const int k = 2560 * half + 512 * c + 8 * lane;
+            float d = 0.f, mul = 0.f;
+            if (MODE != T_F16) quant8_scale_ordered<MODE, X86>(v[c], lane, d, mul);
+            const half8 o = quant8_operand<MODE, X86, true>(v[c], d, mul, down);
+            if (live && k < kp) *reinterpret_cast<half8*>(ar + k) = o;
+        }
+        return;
+    }
 #pragma unroll
     for (int c = 0; c < CHH; ++c) {
         const int k = 2560 * half + 512 * c + 8 * lane;
-        const half8 o = quant8<MODE, X86>(v[c], lane, down);
+        float d = 0.f, mul = 0.f;
+        if (MODE != T_F16) quant8_scale_of<MODE, X86>(ext[c], d, mul);
+        const half8 o = quant8_operand<MODE, X86, false>(v[c], d, mul, down);
         if (live && k < kp) *reinterpret_cast<half8*>(ar + k) = o;
     }
 }
