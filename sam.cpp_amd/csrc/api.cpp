@@ -139,6 +139,7 @@ struct samhip_context {
     bool kq_isum = false;       // SAMHIP_KQ_ISUM=1: the K-quant int8 strip kernel in its integer form (per
                                 // super-block integer sums, ggml's F32 steps in K order: the oracle's bits with
                                 // one K slice; measured 5 % slower on the Q4_K text stream)
+    bool strip16 = true;        // SAMHIP_STRIP16=0 keeps Q4_K / Q5_K products off the packed-activation strip kernel
     int strip_rows = 0;         // SAMHIP_I8_STRIP_ROWS: weight rows per workgroup of the int8 strip kernels,
                                 // 32 or 64 (64 only for K slices of at most 256 values); 0: 64 where that
                                 // brings the grid into one round
@@ -356,6 +357,7 @@ int samhip_context_create(const samhip_options* options, samhip_context** out) {
     ctx->fused_max_splits = std::max(1, env_int("SAMHIP_FUSED_MAX_SPLITS", 16));
     ctx->int8_strip = env_int("SAMHIP_INT8_STRIP", 1);
     ctx->strip_rows = env_int("SAMHIP_I8_STRIP_ROWS", 0);
+    ctx->strip16 = env_int("SAMHIP_STRIP16", 1) != 0;
     ctx->kq_isum = env_int("SAMHIP_KQ_ISUM", 0) != 0;
     ctx->vit_fc1_codes = env_int("SAMHIP_VIT_FC1_CODES", 0) != 0;
     ctx->tall_small = env_int("SAMHIP_TALL_SMALL", 1) != 0;
@@ -555,8 +557,36 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
         std::snprintf(ctx->info.kernel_variant, sizeof(ctx->info.kernel_variant), "%s", variant);
         return SAMHIP_OK;
     }
-    if (!tall && M < kStripMaxM && (w->type == T_Q8_0 || kquant) && ctx->compute == SAMHIP_COMPUTE_Q8_NATIVE &&
-        ctx->int8_strip && ctx->fused_skinny) {
+    const bool int8_rows = !tall && M < kStripMaxM && ctx->compute == SAMHIP_COMPUTE_Q8_NATIVE && ctx->int8_strip &&
+                           ctx->fused_skinny;
+    const bool int8_strip = int8_rows && (w->type == T_Q8_0 || kquant);
+    if (int8_rows && ctx->strip16 && !ctx->kq_isum && strip16_supported(w->type, K, w->data, int64_t(w->nb[1])) &&
+        strip16_preferred(w->type, M, N, K, ctx->cus, kquant)) {
+        // packed activations first, then every workgroup the whole K range;
+        // not where a no-allocation or captured call lacks the scratch
+        const size_t packed = strip16_bytes(M, K);
+        if (packed <= ctx->staging_bytes || !(ctx->no_alloc || ctx->capturing)) {
+            // reserve what the route it replaces would have, too
+            const size_t parts = kquant ? i8_strip_part_bytes(M, N, K, i8_strip_slice_sb(w->type, M, N, K, ctx->cus))
+                                        : fused_skinny_plan(M, N, K, ctx->fused_max_splits, ctx->cus).part_bytes;
+            if (!(ctx->no_alloc || ctx->capturing))
+                if (int rc = ensure_staging(ctx, std::max({packed, parts, size_t(256)}))) return rc;
+            const char* variant = kq_strip_i8_variant(w->type);
+            int rc = traced(ctx, variant, w->type, M, N, K, [&]() -> int {
+                launch_strip16(w->type, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), w->data,
+                               int64_t(w->nb[1]), static_cast<float*>(y->data), int64_t(y->nb[1] / 4), ctx->staging, M,
+                               N, K, ctx->cus, ctx->stream);
+                HIP_TRY(hipGetLastError(), "int8 strip launch");
+                return SAMHIP_OK;
+            });
+            if (rc) return rc;
+            ctx->info.mul_mat_calls++;
+            ctx->info.skinny_launches++;
+            std::snprintf(ctx->info.kernel_variant, sizeof(ctx->info.kernel_variant), "%s", variant);
+            return SAMHIP_OK;
+        }
+    }
+    if (int8_strip) {
         // exact int8 block dots in blocks of 32 activation rows (the text
         // encoder, the decoder's queries and prompt); K slices of 256-1024
         // values, and a reduce launch when there is more than one

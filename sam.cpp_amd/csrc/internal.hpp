@@ -365,6 +365,28 @@ const char* kq_strip_i8_variant(int wtype);
 const char* launch_kq_strip_i8(int wtype, const float* x, int64_t ldx, const void* w, int64_t w_stride, float* y,
                                int64_t ldy, float* part, int M, int N, int K, int slice_sb, bool two_tiles, bool isum,
                                hipStream_t stream);
+// Exact Q4_K / Q5_K products (16-byte aligned weight rows, K > 256) with the
+// activations packed by a launch of their own and the whole K range in each
+// workgroup (strip16.hip); the packed rows go through `scratch`
+// (strip16_bytes).  Taken from 64 workgroups of 16 weight rows x 16
+// activation rows on (fewer leave the chip idle where K slices do not:
+// M = 20, N = 300, K = 4608 8.2 against 7.7 us), except where the one-launch
+// strip kernel needs no reduction for at most 512 values (M = 120, N = 2048,
+// K = 512 7.1 against 6.2 us).  Eager, Q4_K, against the strip kernel with
+// K slices: M = 32, K = 1024, N = 1024 / 3072 / 4096 7.3 / 8.9 / 9.0 ->
+// 6.3 / 6.4 / 6.4 us, M = 64, N = 1024, K = 4096 11.7 -> 8.9; against the
+// fused kernel: M = 100, N = 4736, K = 1024 19.9 -> 15.4, M = 1, N = 4736,
+// K = 4608 15.6 -> 10.5, M = 200, N = 3000, K = 4096 52 -> 43, M = 200,
+// N = 4736, K = 512 22.7 -> 11.5.
+bool strip16_supported(int wtype, int K, const void* w, int64_t w_stride);
+// one_launch: kq_strip_i8_preferred takes the product
+inline bool strip16_preferred(int wtype, int M, int N, int K, int cus, bool one_launch) {
+    if (one_launch && K <= 512 && 256 * i8_strip_slice_sb(wtype, M, N, K, cus) >= K) return false;
+    return int64_t((N + 15) / 16) * ((M + 15) / 16) >= 64;
+}
+size_t strip16_bytes(int M, int K);
+void launch_strip16(int wtype, const float* x, int64_t ldx, const void* w, int64_t w_stride, float* y, int64_t ldy,
+                    void* scratch, int M, int N, int K, int cus, hipStream_t stream);
 const char* strip_skinny_variant(int wtype);
 const char* launch_strip_skinny(int wtype, bool f16, const float* x, int64_t ldx, const void* w, int64_t w_stride,
                                 float* y, int64_t ldy, float* part, int M, int N, int K, int x86, hipStream_t stream);
