@@ -13,12 +13,6 @@
 
 namespace samhip {
 
-
-__device__ __forceinline__ float wave_sum(float v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // ggml_gelu_erf on one F32 value: 0.5 x (1 + erf(x / sqrt 2)), in ggml's
 // order of operations (erf rounded to F32, then 1 + erf).  erf(t) is
 // sign(t) (1 - erfc(a)), a = min(|t|, 4), with
@@ -159,6 +153,20 @@ __device__ __forceinline__ uint32_t umax_xor32(uint32_t v) {
     const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
     return umax(r[0], r[1]);
 }
+// Sum over the wave by the xor butterfly 32, 16, .. 1, on row swaps and DPP
+// (rotations by 8 and 4 reach the xor partner's value, since the values
+// already repeat every 16 and 8 lanes).
+__device__ __forceinline__ float wave_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    v += dpp<DPP_ROR8>(v);
+    v += dpp<DPP_ROR4>(v);
+    v += dpp<DPP_XOR2>(v);
+    return v + dpp<DPP_XOR1>(v);
+}
+
 typedef float floatx8 __attribute__((ext_vector_type(8)));
 
 // x / 127 correctly rounded for x >= 0 (a Q8_0 block maximum): the product

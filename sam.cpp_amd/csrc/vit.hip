@@ -17,6 +17,7 @@
 #include <algorithm>
 
 #include "internal.hpp"
+#include "q8stage.hpp"
 
 #pragma clang fp contract(off)
 
@@ -28,12 +29,14 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ float wave_sum(float v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 __device__ __forceinline__ floatx4 ld4(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
+// four floats at a 4-byte aligned address
+__device__ __forceinline__ floatx4 ld4a(const float* p) {
+    struct __attribute__((packed, aligned(4))) unaligned4 {
+        floatx4 v;
+    };
+    return reinterpret_cast<const unaligned4*>(p)->v;
+}
 
 // ---------------------------------------------------------------------------
 // Layer norm: one wave per row of E = 256 * CH floats.
@@ -51,18 +54,32 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float* __restrict
     const float* xr = x + int64_t(r) * E;
     const float* ar = add ? add + int64_t((gy % add_grid) * add_grid + gx % add_grid) * E : nullptr;
     floatx4 v[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) v[c] = ld4(xr + 256 * c + 4 * lane);
+    // every load is requested before the reductions (element by element
+    // behind null tests, a row waited for them one after another: 5184 rows of
+    // 1024 floats 20.6 -> 11.8 us, 3.6 TB/s)
+    floatx4 wv[CH], bv[CH];
+    if (w)
+#pragma unroll
+        for (int c = 0; c < CH; ++c) wv[c] = ld4a(w + 256 * c + 4 * lane);
+    if (b)
+#pragma unroll
+        for (int c = 0; c < CH; ++c) bv[c] = ld4a(b + 256 * c + 4 * lane);
+    if (ar) {
+        floatx4 a[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) a[c] = ld4(ar + 256 * c + 4 * lane);
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[c][i] = v[c][i] + a[c][i];
+    }
     float s = 0.f;
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        v[c] = ld4(xr + 256 * c + 4 * lane);
-        if (ar) {
-            const floatx4 a = ld4(ar + 256 * c + 4 * lane);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[c][i] = v[c][i] + a[i];
-        }
+    for (int c = 0; c < CH; ++c)
 #pragma unroll
         for (int i = 0; i < 4; ++i) s += v[c][i];
-    }
     const float mean = wave_sum(s) / float(E);
     float s2 = 0.f;
 #pragma unroll
@@ -83,16 +100,16 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float* __restrict
     float* yr = y + dst * E;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-        const int k = 256 * c + 4 * lane;
-        floatx4 o;
+        floatx4 o = v[c];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float t = v[c][i] * scale;
-            if (w) t = t * w[k + i];
-            if (b) t = t + b[k + i];
-            o[i] = t;
-        }
-        *reinterpret_cast<floatx4*>(yr + k) = o;
+        for (int i = 0; i < 4; ++i) o[i] = o[i] * scale;
+        if (w)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = o[i] * wv[c][i];
+        if (b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = o[i] + bv[c][i];
+        *reinterpret_cast<floatx4*>(yr + 256 * c + 4 * lane) = o;
     }
 }
 
