@@ -115,7 +115,11 @@ struct samhip_context {
     // path, the call's fp16 weights [N][K]
     void* staging = nullptr;
     size_t staging_bytes = 0;
-    int* flag = nullptr;   // device error flag (get_rows id range)
+    int* flag = nullptr;   // device error flag (activation range)
+    // get_rows' id range flag in pinned host memory: the kernel stores to it
+    // directly, so the call is one launch and a stream wait (a device flag
+    // took a fill before and a copy after it: 15 us more a call)
+    int* host_flag = nullptr;
     // this device's fixed scratch (samhip_mul_mat_noalloc); while such a call
     // runs, `staging` points at it and `no_alloc` forbids growing it
     void* fixed_scratch = nullptr;
@@ -338,7 +342,8 @@ int samhip_context_create(const samhip_options* options, samhip_context** out) {
     hipDeviceProp_t prop;
     if (hipSetDevice(o.device) != hipSuccess || hipGetDeviceProperties(&prop, o.device) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void**>(&ctx->flag), sizeof(int)) != hipSuccess) {
+        hipMalloc(reinterpret_cast<void**>(&ctx->flag), sizeof(int)) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&ctx->host_flag), sizeof(int), hipHostMallocCoherent) != hipSuccess) {
         samhip_context_destroy(ctx);
         return fail(SAMHIP_ERR_DEVICE, "HIP context initialization failed");
     }
@@ -384,6 +389,7 @@ void samhip_context_destroy(samhip_context* ctx) {
     if (ctx->row_map) (void)hipFree(ctx->row_map);
     for (void* p : ctx->retired_staging) (void)hipFree(p);
     if (ctx->flag) (void)hipFree(ctx->flag);
+    if (ctx->host_flag) (void)hipHostFree(ctx->host_flag);
     for (auto& r : ctx->trace) {
         (void)hipEventDestroy(r.start);
         (void)hipEventDestroy(r.stop);
@@ -812,13 +818,15 @@ int samhip_get_rows(samhip_context* ctx, const samhip_tensor* src, const samhip_
     for (int i = 2; i < 4; ++i)
         if (src->ne[i] != 1 || ids->ne[i] != 1 || dst->ne[i] != 1) return fail(SAMHIP_ERR_INVALID_ARGUMENT, "get_rows: 2-D only");
     if (int rc = set_device(ctx)) return rc;
-    HIP_TRY(hipMemsetAsync(ctx->flag, 0, sizeof(int), ctx->stream), "hipMemsetAsync");
+    // no kernel of an earlier call is in flight: each waited for its own
+    volatile int* const bad_id = ctx->host_flag;
+    *bad_id = 0;
     launch_dequant_rows(t, src->data, int64_t(src->nb[1]), static_cast<const int32_t*>(ids->data), rows,
-                        static_cast<float*>(dst->data), int64_t(dst->nb[1] / 4), int(n), int(K), ctx->flag, ctx->stream);
+                        static_cast<float*>(dst->data), int64_t(dst->nb[1] / 4), int(n), int(K), ctx->host_flag,
+                        ctx->stream);
     HIP_TRY(hipGetLastError(), "get_rows launch");
-    int bad = 0;
-    HIP_TRY(hipMemcpyAsync(&bad, ctx->flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
     HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    const int bad = *bad_id;
     ctx->info.get_rows_calls++;
     if (bad) return fail(SAMHIP_ERR_INVALID_ARGUMENT, "get_rows: row id out of range [0, %lld)", (long long)rows);
     return SAMHIP_OK;

@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(const uint8_t* __rest
         if (ids) {
             sr = ids[r];
             if (sr < 0 || sr >= src_rows) {
-                if (c == 0) atomicOr(bad_id, 1);
+                if (c == 0) *bad_id = 1;   // (host memory: a plain store, every writer's the same)
                 continue;
             }
         }
