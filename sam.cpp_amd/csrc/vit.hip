@@ -346,6 +346,9 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
         floatx16 s0, s1;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s0[r] = s1[r] = 0.f;
+        // the wave with products to issue goes before those in their softmax
+        // (a Q8_0 block with global attention 605 -> 602 us)
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             // rows li and 32 + li, chunk 2s + hh (same swizzle: (32 + li) & 7 == li & 7)
@@ -365,6 +368,7 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
                 s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qf[P - 1][s], s1, 0, 0, 0);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         // keys past N (only in the last tile)
         const int kbase = kb * 64;
         if (kbase + 64 > N) {
@@ -451,6 +455,7 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
             else wait_vmcnt0();
             __syncthreads();
         }
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             half8 a0, a1;
@@ -466,6 +471,7 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
                 o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(l1, pf[0][u], o1, 0, 0, 0);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         if (kb + 1 < kb1) {
             wait_vmcnt0();   // this wave's loads of the next tile landed
             __syncthreads();
