@@ -368,21 +368,26 @@ const char* launch_kq_strip_i8(int wtype, const float* x, int64_t ldx, const voi
 // Exact Q4_K / Q5_K products (16-byte aligned weight rows, K > 256) with the
 // activations packed by a launch of their own and the whole K range in each
 // workgroup (strip16.hip); the packed rows go through `scratch`
-// (strip16_bytes).  Taken from 64 workgroups of 16 weight rows x 16
-// activation rows on (fewer leave the chip idle where K slices do not:
-// M = 20, N = 300, K = 4608 8.2 against 7.7 us), except where the one-launch
-// strip kernel needs no reduction for at most 512 values (M = 120, N = 2048,
-// K = 512 7.1 against 6.2 us).  Eager, Q4_K, against the strip kernel with
-// K slices: M = 32, K = 1024, N = 1024 / 3072 / 4096 7.3 / 8.9 / 9.0 ->
-// 6.3 / 6.4 / 6.4 us, M = 64, N = 1024, K = 4096 11.7 -> 8.9; against the
-// fused kernel: M = 100, N = 4736, K = 1024 19.9 -> 15.4, M = 1, N = 4736,
-// K = 4608 15.6 -> 10.5, M = 200, N = 3000, K = 4096 52 -> 43, M = 200,
-// N = 4736, K = 512 22.7 -> 11.5.
+// (strip16_bytes).  Eager, Q4_K, one box, against the K-sliced strip kernel:
+// M = 32, K = 1024, N = 1024 / 3072 / 4096 7.3 / 8.9 / 9.0 -> 6.3 / 6.4 / 6.4
+// us; M = 128, N = 1024, K = 1536 11.6 -> 7.6; against the fused kernel:
+// M = 200, N = 4096, K = 512 17.2 -> 10.4, M = 100, N = 4736, K = 1024 19.9 ->
+// 15.4, M = 1, N = 4736, K = 4608 15.6 -> 10.5.
 bool strip16_supported(int wtype, int K, const void* w, int64_t w_stride);
-// one_launch: kq_strip_i8_preferred takes the product
+// Where it measured slower, over M = 1 .. 255, N = 100 .. 4096, K = 512 ..
+// 4096:
+//   * fewer than 64 workgroups of 16 x 16 rows (128 past K = 1024), which
+//     leave the chip idle where K slices do not: M = 200, N = 100, K = 4096
+//     9.9 against 8.7 us, M = 32, N = 512, K = 4096 8.4 against 7.8;
+//   * short K that the strip kernel takes in one launch without a reduction
+//     (one_launch: kq_strip_i8_preferred takes the product): M = 200,
+//     N = 1024, K = 768 8.3 against 7.6;
+//   * more than seven workgroups of 16 x 32 rows per CU: M = 255, N = 4096,
+//     K = 1024 22.0 against the fused kernel's 18.0 (M = 200: 19.6, 22.8).
 inline bool strip16_preferred(int wtype, int M, int N, int K, int cus, bool one_launch) {
-    if (one_launch && K <= 512 && 256 * i8_strip_slice_sb(wtype, M, N, K, cus) >= K) return false;
-    return int64_t((N + 15) / 16) * ((M + 15) / 16) >= 64;
+    if (one_launch && K < 1024 && 256 * i8_strip_slice_sb(wtype, M, N, K, cus) >= K) return false;
+    const int64_t rg = (N + 15) / 16, tiles = (M + 15) / 16;
+    return rg * tiles >= (K > 1024 ? 128 : 64) && rg * ((tiles + 1) / 2) <= 7 * int64_t(cus);
 }
 size_t strip16_bytes(int M, int K);
 void launch_strip16(int wtype, const float* x, int64_t ldx, const void* w, int64_t w_stride, float* y, int64_t ldy,

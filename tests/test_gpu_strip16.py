@@ -18,8 +18,9 @@ def row_rel(y, ref):
     return (np.linalg.norm(y.astype(np.float64) - ref, axis=1) / np.maximum(np.linalg.norm(ref.astype(np.float64), axis=1), 1e-30)).max()
 
 
-SHAPES = [(1, 1024, 512, None), (15, 1030, 768, 769), (16, 1024, 1024, None), (17, 517, 1280, None), (33, 400, 2048, 2052),
-          (49, 257, 2304, None), (255, 70, 4096, None), (100, 4733, 1024, None), (31, 4096, 4608, None)]
+# (each has at least 128 workgroups of 16 x 16 rows, or 64 up to K = 1024, and is past one launch of the strip kernel)
+SHAPES = [(100, 2100, 512, None), (15, 1030, 768, 769), (16, 1024, 1024, None), (17, 1030, 1280, None), (33, 700, 2048, 2052),
+          (49, 517, 2304, None), (255, 130, 4096, None), (100, 4733, 1024, None), (31, 4096, 4608, None), (1, 2064, 2048, None)]
 
 
 @pytest.mark.parametrize("qtype", [12, 13])
