@@ -732,16 +732,22 @@ void launch_quantize_act(int type, const float* x, int64_t x_stride, int rows, i
         return;
     }
     const int nb = K / 32;
-    const int64_t blocks = int64_t(rows) * nb;
-    const dim3 grid(unsigned((blocks + 4 * kQ8WaveBlocks - 1) / (4 * kQ8WaveBlocks)));
     const bool xvec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && x_stride % 4 == 0;
+    // (a dispatch counts its work-items in 32 bits: four per block here)
+    const int step = int(std::max<int64_t>(1, (int64_t(1) << 28) / nb));
+    for (int64_t r0 = 0; r0 < rows; r0 += step) {
+        const int64_t blocks = std::min<int64_t>(step, rows - r0) * nb;
+        const dim3 grid(unsigned((blocks + 4 * kQ8WaveBlocks - 1) / (4 * kQ8WaveBlocks)));
+        const float* xs = x + r0 * x_stride;
+        uint8_t* ds = d + r0 * nb * 34;
 #define SAMHIP_Q8_0(X86, XVEC) \
-    hipLaunchKernelGGL((quantize_q8_0_kernel<X86, XVEC>), grid, dim3(256), 0, stream, x, x_stride, blocks, nb, d)
-    if (x86 && xvec) SAMHIP_Q8_0(true, true);
-    else if (x86) SAMHIP_Q8_0(true, false);
-    else if (xvec) SAMHIP_Q8_0(false, true);
-    else SAMHIP_Q8_0(false, false);
+    hipLaunchKernelGGL((quantize_q8_0_kernel<X86, XVEC>), grid, dim3(256), 0, stream, xs, x_stride, blocks, nb, ds)
+        if (x86 && xvec) SAMHIP_Q8_0(true, true);
+        else if (x86) SAMHIP_Q8_0(true, false);
+        else if (xvec) SAMHIP_Q8_0(false, true);
+        else SAMHIP_Q8_0(false, false);
 #undef SAMHIP_Q8_0
+    }
 }
 
 // ---------------------------------------------------------------------------
