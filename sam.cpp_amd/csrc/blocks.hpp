@@ -43,6 +43,18 @@ __device__ __forceinline__ uint16_t float_to_half_bits(float f) {
     return __builtin_bit_cast(uint16_t, (_Float16)f);
 }
 
+// Between one lane's LDS stores and another lane's loads of the same wave.
+// The wave's LDS operations execute in order; the fences keep the compiler
+// from moving either side across (s_waitcnt and wave_barrier alone are no
+// memory operations to it, and with two access types it may take the loads
+// for unrelated).  They emit no instruction at this scope.
+__device__ __forceinline__ void wave_lds_handoff() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ({hi, lo} >> 8*shift)[31:0]
 __device__ __forceinline__ uint32_t funnel_bytes(uint32_t hi, uint32_t lo, uint32_t shift) {
     return __builtin_amdgcn_alignbyte(hi, lo, shift);

@@ -443,8 +443,7 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restr
     if ((lane & 3) == 0) o[0] = float_to_half_bits(d);
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[1 + 4 * (lane & 3) + j] = uint16_t((q[2 * j] & 0xff) | ((q[2 * j + 1] & 0xff) << 8));
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the wave's bytes are in LDS
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_handoff();   // 16-bit stores above, 32-bit loads below
     const int bytes = int(min(int64_t(kQ8WaveBlocks), blocks - first)) * 34;
     uint8_t* out = dst + first * 34;
     if (reinterpret_cast<uintptr_t>(dst) % 4 == 0) {

@@ -177,8 +177,7 @@ __global__ __launch_bounds__(64 * NW) void strip16_kernel(const int8_t* __restri
             for (int l = 0; l < SL; ++l)
                 if (32 * U % 64 == 0 || lane < 32 * U) (&rowv[wave][t][1][0])[64 * l + lane] = sv[t][l];
         }
-        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the wave's own row vectors are in LDS
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_handoff();   // the wave's own row vectors
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -201,7 +200,7 @@ __global__ __launch_bounds__(64 * NW) void strip16_kernel(const int8_t* __restri
                     }
                 }
             }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_handoff();   // read before the next run's are stored
     }
 #pragma unroll
     for (int t = 0; t < T; ++t)
