@@ -120,6 +120,10 @@ struct samhip_context {
     // directly, so the call is one launch and a stream wait (a device flag
     // took a fill before and a copy after it: 15 us more a call)
     int* host_flag = nullptr;
+    // strip16's packed activation rows (kStrip16Bytes, for the context's life):
+    // not part of `staging`, so that which kernel a product runs on follows
+    // from its operands alone, in a capture too
+    void* packed_rows = nullptr;
     // this device's fixed scratch (samhip_mul_mat_noalloc); while such a call
     // runs, `staging` points at it and `no_alloc` forbids growing it
     void* fixed_scratch = nullptr;
@@ -343,7 +347,8 @@ int samhip_context_create(const samhip_options* options, samhip_context** out) {
     if (hipSetDevice(o.device) != hipSuccess || hipGetDeviceProperties(&prop, o.device) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc(reinterpret_cast<void**>(&ctx->flag), sizeof(int)) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&ctx->host_flag), sizeof(int), hipHostMallocCoherent) != hipSuccess) {
+        hipHostMalloc(reinterpret_cast<void**>(&ctx->host_flag), sizeof(int), hipHostMallocCoherent) != hipSuccess ||
+        hipMalloc(&ctx->packed_rows, kStrip16Bytes) != hipSuccess) {
         samhip_context_destroy(ctx);
         return fail(SAMHIP_ERR_DEVICE, "HIP context initialization failed");
     }
@@ -390,6 +395,7 @@ void samhip_context_destroy(samhip_context* ctx) {
     for (void* p : ctx->retired_staging) (void)hipFree(p);
     if (ctx->flag) (void)hipFree(ctx->flag);
     if (ctx->host_flag) (void)hipHostFree(ctx->host_flag);
+    if (ctx->packed_rows) (void)hipFree(ctx->packed_rows);
     for (auto& r : ctx->trace) {
         (void)hipEventDestroy(r.start);
         (void)hipEventDestroy(r.stop);
@@ -566,31 +572,31 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     const bool int8_rows = !tall && M < kStripMaxM && ctx->compute == SAMHIP_COMPUTE_Q8_NATIVE && ctx->int8_strip &&
                            ctx->fused_skinny;
     const bool int8_strip = int8_rows && (w->type == T_Q8_0 || kquant);
-    if (int8_rows && ctx->strip16 && !ctx->kq_isum && strip16_supported(w->type, K, w->data, int64_t(w->nb[1])) &&
+    if (int8_rows && ctx->strip16 && !ctx->kq_isum && strip16_supported(w->type, M, K, w->data, int64_t(w->nb[1])) &&
         strip16_preferred(w->type, M, N, K, ctx->cus, kquant)) {
-        // packed activations first, then every workgroup the whole K range;
-        // not where a no-allocation or captured call lacks the scratch
-        const size_t packed = strip16_bytes(M, K);
-        if (packed <= ctx->staging_bytes || !(ctx->no_alloc || ctx->capturing)) {
-            // reserve what the route it replaces would have, too
-            const size_t parts = kquant ? i8_strip_part_bytes(M, N, K, i8_strip_slice_sb(w->type, M, N, K, ctx->cus))
-                                        : fused_skinny_plan(M, N, K, ctx->fused_max_splits, ctx->cus).part_bytes;
-            if (!(ctx->no_alloc || ctx->capturing))
-                if (int rc = ensure_staging(ctx, std::max({packed, parts, size_t(256)}))) return rc;
-            const char* variant = kq_strip_i8_variant(w->type);
-            int rc = traced(ctx, variant, w->type, M, N, K, [&]() -> int {
-                launch_strip16(w->type, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), w->data,
-                               int64_t(w->nb[1]), static_cast<float*>(y->data), int64_t(y->nb[1] / 4), ctx->staging, M,
-                               N, K, ctx->cus, ctx->stream);
-                HIP_TRY(hipGetLastError(), "int8 strip launch");
-                return SAMHIP_OK;
-            });
-            if (rc) return rc;
-            ctx->info.mul_mat_calls++;
-            ctx->info.skinny_launches++;
-            std::snprintf(ctx->info.kernel_variant, sizeof(ctx->info.kernel_variant), "%s", variant);
+        // packed activations first, then every workgroup the whole K range.
+        // The packed rows have their own place (in a no-allocation call the
+        // fixed scratch, which holds them); the staging asked for here is
+        // what the route for rows that are not 16-byte aligned reserves, so a
+        // capture is refused before anything has run, whatever the alignment.
+        const size_t parts = kquant ? i8_strip_part_bytes(M, N, K, i8_strip_slice_sb(w->type, M, N, K, ctx->cus))
+                                    : fused_skinny_plan(M, N, K, ctx->fused_max_splits, ctx->cus).part_bytes;
+        const size_t reserve = std::max(parts, size_t(256));
+        if (int rc = ensure_staging(ctx, ctx->capturing ? std::min(reserve, strip16_bytes(M, K)) : reserve)) return rc;
+        void* const scratch = ctx->no_alloc ? ctx->staging : ctx->packed_rows;
+        const char* variant = kq_strip_i8_variant(w->type);
+        int rc = traced(ctx, variant, w->type, M, N, K, [&]() -> int {
+            launch_strip16(w->type, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), w->data,
+                           int64_t(w->nb[1]), static_cast<float*>(y->data), int64_t(y->nb[1] / 4), scratch, M, N, K,
+                           ctx->cus, ctx->stream);
+            HIP_TRY(hipGetLastError(), "int8 strip launch");
             return SAMHIP_OK;
-        }
+        });
+        if (rc) return rc;
+        ctx->info.mul_mat_calls++;
+        ctx->info.skinny_launches++;
+        std::snprintf(ctx->info.kernel_variant, sizeof(ctx->info.kernel_variant), "%s", variant);
+        return SAMHIP_OK;
     }
     if (int8_strip) {
         // exact int8 block dots in blocks of 32 activation rows (the text

@@ -373,7 +373,10 @@ const char* launch_kq_strip_i8(int wtype, const float* x, int64_t ldx, const voi
 // us; M = 128, N = 1024, K = 1536 11.6 -> 7.6; against the fused kernel:
 // M = 200, N = 4096, K = 512 17.2 -> 10.4, M = 100, N = 4736, K = 1024 19.9 ->
 // 15.4, M = 1, N = 4736, K = 4608 15.6 -> 10.5.
-bool strip16_supported(int wtype, int K, const void* w, int64_t w_stride);
+// strip16_supported: also that the packed rows fit kStrip16Bytes (255 rows of
+// 57 000 values, 32 of 460 000).
+constexpr size_t kStrip16Bytes = size_t(16) << 20;
+bool strip16_supported(int wtype, int M, int K, const void* w, int64_t w_stride);
 // Where it measured slower, over M = 1 .. 255, N = 100 .. 4096, K = 512 ..
 // 4096:
 //   * fewer than 64 workgroups of 16 x 16 rows (128 past K = 1024), which

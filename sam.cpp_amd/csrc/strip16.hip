@@ -220,12 +220,12 @@ __global__ __launch_bounds__(64 * NW) void strip16_kernel(const int8_t* __restri
 
 }  // namespace
 
-bool strip16_supported(int wtype, int K, const void* w, int64_t w_stride) {
-    return (wtype == T_Q4_K || wtype == T_Q5_K) && K > 256 && K % 256 == 0 &&
+size_t strip16_bytes(int M, int K) { return packed_rows(M, K).bytes; }
+
+bool strip16_supported(int wtype, int M, int K, const void* w, int64_t w_stride) {
+    return (wtype == T_Q4_K || wtype == T_Q5_K) && K > 256 && K % 256 == 0 && strip16_bytes(M, K) <= kStrip16Bytes &&
            reinterpret_cast<uintptr_t>(w) % 16 == 0 && w_stride % 16 == 0;
 }
-
-size_t strip16_bytes(int M, int K) { return packed_rows(M, K).bytes; }
 
 void launch_strip16(int wtype, const float* x, int64_t ldx, const void* w, int64_t w_stride, float* y, int64_t ldy,
                     void* scratch, int M, int N, int K, int cus, hipStream_t stream) {

@@ -100,3 +100,41 @@ def test_strip16_capture_and_noalloc(samhip, oracle):
             ctx.mul_mat(samhip.tensor(13, k, n, wb.ptr), samhip.tensor(samhip.F32, k, m, xb.ptr),
                         samhip.tensor(samhip.F32, n, m, yb.ptr))
         ctx.capture_end().destroy()
+
+
+@pytest.mark.parametrize("m,n,k", [(255, 130, 4096), (255, 512, 32768)])
+def test_strip16_arithmetic_does_not_depend_on_earlier_calls(samhip, oracle, m, n, k):
+    """A capture in a context that has only run other products and the
+    no-allocation entry give the eager call's bits: those products leave less
+    staging than the packed rows take (1.2 and 9.5 MB), but enough for the
+    kernels that would otherwise stand in, the exact one with another order
+    of sums and the one that rounds its operands to fp16."""
+    print("case strip16 history", m, n, k, flush=True)
+    rng = np.random.default_rng(n + k)
+    w = oracle.quantize(12, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    rows = [0, 1, m // 2, m - 1]
+    ref = oracle.mul_mat_native(12, w, np.ascontiguousarray(x[rows]))
+    with samhip.Context(0) as ctx:
+        eager = ctx.matmul(12, w, x)
+    assert row_rel(eager[rows], ref) <= EXACT
+    with samhip.Context(0) as ctx:
+        if k > 4096:   # 5 MB
+            ctx.matmul(8, oracle.quantize(8, np.ones((512, 1024), np.float32)), np.ones((2000, 1024), np.float32))
+        else:          # 1 MB
+            ctx.matmul(12, w[:64, :144], np.ascontiguousarray(x[:4, :256]))
+        assert ctx.query().activation_allocation_peak_bytes < 256 * k * 9 // 8
+        wb, xb, yb = ctx.upload(w), ctx.upload(x), ctx.alloc(m * n * 4)
+        W, X, Y = samhip.tensor(12, k, n, wb.ptr), samhip.tensor(samhip.F32, k, m, xb.ptr), samhip.tensor(samhip.F32, n, m, yb.ptr)
+        ctx.capture_begin()
+        ctx.mul_mat(W, X, Y)
+        graph = ctx.capture_end()
+        for _ in range(2):
+            ctx.write(yb, np.zeros((m, n), np.float32))
+            graph.launch()
+            ctx.synchronize()
+            assert np.array_equal(ctx.download(yb, (m, n), np.float32).view(np.uint32), eager.view(np.uint32))
+        graph.destroy()
+        ctx.write(yb, np.zeros((m, n), np.float32))
+        samhip.check(samhip.lib().samhip_mul_mat_noalloc(ctx.handle, ctypes.byref(W), ctypes.byref(X), ctypes.byref(Y)))
+        assert np.array_equal(ctx.download(yb, (m, n), np.float32).view(np.uint32), eager.view(np.uint32))
