@@ -148,6 +148,7 @@ struct samhip_context {
                                 // super-block integer sums, ggml's F32 steps in K order: the oracle's bits with
                                 // one K slice; measured 5 % slower on the Q4_K text stream)
     bool strip16 = true;        // SAMHIP_STRIP16=0 keeps Q4_K / Q5_K products off the packed-activation strip kernel
+                                // (as do INT8_STRIP=2, I8_STRIP_ROWS, KQ_ISUM and STRIP_SKINNY=2, which ask for others)
     int strip_rows = 0;         // SAMHIP_I8_STRIP_ROWS: weight rows per workgroup of the int8 strip kernels,
                                 // 32 or 64 (64 only for K slices of at most 256 values); 0: 64 where that
                                 // brings the grid into one round
@@ -572,7 +573,10 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     const bool int8_rows = !tall && M < kStripMaxM && ctx->compute == SAMHIP_COMPUTE_Q8_NATIVE && ctx->int8_strip &&
                            ctx->fused_skinny;
     const bool int8_strip = int8_rows && (w->type == T_Q8_0 || kquant);
-    if (int8_rows && ctx->strip16 && !ctx->kq_isum && strip16_supported(w->type, M, K, w->data, int64_t(w->nb[1])) &&
+    // (a setting that asks for one of the one-launch strip kernels gets it)
+    const bool strip16 = ctx->strip16 && ctx->int8_strip == 1 && ctx->strip_rows == 0 && !ctx->kq_isum &&
+                         ctx->strip_skinny != 2;
+    if (int8_rows && strip16 && strip16_supported(w->type, M, K, w->data, int64_t(w->nb[1])) &&
         strip16_preferred(w->type, M, N, K, ctx->cus, kquant)) {
         // packed activations first, then every workgroup the whole K range.
         // The packed rows have their own place (in a no-allocation call the

@@ -138,3 +138,28 @@ def test_strip16_arithmetic_does_not_depend_on_earlier_calls(samhip, oracle, m, 
         ctx.write(yb, np.zeros((m, n), np.float32))
         samhip.check(samhip.lib().samhip_mul_mat_noalloc(ctx.handle, ctypes.byref(W), ctypes.byref(X), ctypes.byref(Y)))
         assert np.array_equal(ctx.download(yb, (m, n), np.float32).view(np.uint32), eager.view(np.uint32))
+
+
+@pytest.mark.parametrize("name,value", [("SAMHIP_INT8_STRIP", "2"), ("SAMHIP_I8_STRIP_ROWS", "32"),
+                                        ("SAMHIP_STRIP_SKINNY", "2")])
+def test_settings_for_the_strip_kernel_reach_it(samhip, oracle, monkeypatch, name, value):
+    """The settings that ask for the one-launch strip kernels give the bits of
+    the one that takes this size (its order of sums differs), not those of
+    the kernel that is the default."""
+    print("case strip settings", name, value, flush=True)
+    m, n, k = 32, 1024, 4096
+    rng = np.random.default_rng(12)
+    w = oracle.quantize(12, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+
+    def run():
+        with samhip.Context(0) as ctx:
+            return ctx.matmul(12, w, x).view(np.uint32)
+
+    default = run()
+    monkeypatch.setenv("SAMHIP_STRIP16", "0")
+    strip = run()
+    assert not np.array_equal(default, strip)   # else the next line says nothing
+    monkeypatch.delenv("SAMHIP_STRIP16")
+    monkeypatch.setenv(name, value)
+    assert np.array_equal(run(), strip)
