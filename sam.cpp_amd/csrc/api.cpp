@@ -587,12 +587,18 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
                                     : fused_skinny_plan(M, N, K, ctx->fused_max_splits, ctx->cus).part_bytes;
         const size_t reserve = std::max(parts, size_t(256));
         if (int rc = ensure_staging(ctx, ctx->capturing ? std::min(reserve, strip16_bytes(M, K)) : reserve)) return rc;
+        static_assert(kStrip16Bytes <= kNoAllocScratchBytes, "the fixed scratch holds the packed rows");
         void* const scratch = ctx->no_alloc ? ctx->staging : ctx->packed_rows;
-        const char* variant = kq_strip_i8_variant(w->type);
-        int rc = traced(ctx, variant, w->type, M, N, K, [&]() -> int {
-            launch_strip16(w->type, static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), w->data,
-                           int64_t(w->nb[1]), static_cast<float*>(y->data), int64_t(y->nb[1] / 4), scratch, M, N, K,
-                           ctx->cus, ctx->stream);
+        const char* variant = strip16_variant(w->type);
+        int rc = traced(ctx, "stage_strip_q8_k", w->type, M, N, K, [&]() -> int {
+            launch_strip16_pack(static_cast<const float*>(x->data), int64_t(x->nb[1] / 4), scratch, M, K, ctx->stream);
+            HIP_TRY(hipGetLastError(), "activation packing launch");
+            return SAMHIP_OK;
+        });
+        if (rc) return rc;
+        rc = traced(ctx, variant, w->type, M, N, K, [&]() -> int {
+            launch_strip16(w->type, scratch, w->data, int64_t(w->nb[1]), static_cast<float*>(y->data),
+                           int64_t(y->nb[1] / 4), M, N, K, ctx->cus, ctx->stream);
             HIP_TRY(hipGetLastError(), "int8 strip launch");
             return SAMHIP_OK;
         });

@@ -393,8 +393,10 @@ inline bool strip16_preferred(int wtype, int M, int N, int K, int cus, bool one_
     return rg * tiles >= (K > 1024 ? 128 : 64) && rg * ((tiles + 1) / 2) <= 7 * int64_t(cus);
 }
 size_t strip16_bytes(int M, int K);
-void launch_strip16(int wtype, const float* x, int64_t ldx, const void* w, int64_t w_stride, float* y, int64_t ldy,
-                    void* scratch, int M, int N, int K, int cus, hipStream_t stream);
+const char* strip16_variant(int wtype);
+void launch_strip16_pack(const float* x, int64_t ldx, void* scratch, int M, int K, hipStream_t stream);
+void launch_strip16(int wtype, const void* scratch, const void* w, int64_t w_stride, float* y, int64_t ldy, int M, int N,
+                    int K, int cus, hipStream_t stream);
 const char* strip_skinny_variant(int wtype);
 const char* launch_strip_skinny(int wtype, bool f16, const float* x, int64_t ldx, const void* w, int64_t w_stride,
                                 float* y, int64_t ldy, float* part, int M, int N, int K, int x86, hipStream_t stream);

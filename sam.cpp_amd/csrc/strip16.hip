@@ -227,21 +227,29 @@ bool strip16_supported(int wtype, int M, int K, const void* w, int64_t w_stride)
            reinterpret_cast<uintptr_t>(w) % 16 == 0 && w_stride % 16 == 0;
 }
 
-void launch_strip16(int wtype, const float* x, int64_t ldx, const void* w, int64_t w_stride, float* y, int64_t ldy,
-                    void* scratch, int M, int N, int K, int cus, hipStream_t stream) {
+const char* strip16_variant(int wtype) { return wtype == T_Q4_K ? "skinny_i8mfma16_q4_k" : "skinny_i8mfma16_q5_k"; }
+
+void launch_strip16_pack(const float* x, int64_t ldx, void* scratch, int M, int K, hipStream_t stream) {
     const PackedRows pr = packed_rows(M, K);
     int8_t* codes = static_cast<int8_t*>(scratch);
     float* scales = reinterpret_cast<float*>(codes + pr.scale_at);
     float* sums = reinterpret_cast<float*>(codes + pr.sum_at);
-    const uint8_t* wb = static_cast<const uint8_t*>(w);
-    const int nsb = K / 256, units = (M + 31) / 32 * 32 * nsb, RG = (N + 15) / 16;
-    const dim3 pgrid(unsigned((units + 7) / 8));
+    const int nsb = K / 256, units = (M + 31) / 32 * 32 * nsb;
+    const dim3 grid(unsigned((units + 7) / 8)), block(256);
     if (reinterpret_cast<uintptr_t>(x) % 16 == 0 && ldx % 4 == 0)
-        hipLaunchKernelGGL(strip_pack_kernel<true>, pgrid, dim3(256), 0, stream, x, ldx, M, nsb, units, codes,
-                           scales, sums);
+        hipLaunchKernelGGL(strip_pack_kernel<true>, grid, block, 0, stream, x, ldx, M, nsb, units, codes, scales, sums);
     else
-        hipLaunchKernelGGL(strip_pack_kernel<false>, pgrid, dim3(256), 0, stream, x, ldx, M, nsb, units, codes,
-                           scales, sums);
+        hipLaunchKernelGGL(strip_pack_kernel<false>, grid, block, 0, stream, x, ldx, M, nsb, units, codes, scales, sums);
+}
+
+void launch_strip16(int wtype, const void* scratch, const void* w, int64_t w_stride, float* y, int64_t ldy, int M, int N,
+                    int K, int cus, hipStream_t stream) {
+    const PackedRows pr = packed_rows(M, K);
+    const int8_t* codes = static_cast<const int8_t*>(scratch);
+    const float* scales = reinterpret_cast<const float*>(codes + pr.scale_at);
+    const float* sums = reinterpret_cast<const float*>(codes + pr.sum_at);
+    const uint8_t* wb = static_cast<const uint8_t*>(w);
+    const int nsb = K / 256, RG = (N + 15) / 16;
     // two row tiles per workgroup share its weight; one while that still
     // leaves every workgroup a CU (and for 16 rows and fewer)
     const int tiles = (M + 15) / 16, pairs = 4 * nsb;

@@ -12,6 +12,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 EXACT = 2e-5
+VARIANT = {12: b"skinny_i8mfma16_q4_k", 13: b"skinny_i8mfma16_q5_k"}
 
 
 def row_rel(y, ref):
@@ -33,8 +34,10 @@ def test_strip16(samhip, oracle, qtype, m, n, k, stride):
     x[0, 3] = np.nan                # packs as code 0
     with samhip.Context(0) as ctx:
         y = ctx.matmul(qtype, w, x, x_row_stride=stride)
-        assert ctx.query().kernel_variant in (b"skinny_i8mfma_q4_k", b"skinny_i8mfma_q5_k")
+        assert ctx.query().kernel_variant == VARIANT[qtype]
+        ctx.trace_begin()
         again = ctx.matmul(qtype, w, x)
+        assert [r[0] for r in ctx.trace_end()] == ["stage_strip_q8_k", VARIANT[qtype].decode()]
     ref = oracle.mul_mat_native(qtype, w, x)
     assert np.isfinite(ref).all() and np.isfinite(y).all() and row_rel(y, ref) <= EXACT
     assert np.array_equal(y.view(np.uint32), again.view(np.uint32))
@@ -59,6 +62,7 @@ def test_strip16_rows_off_alignment_and_guarded_output(samhip, oracle):
             yb = ctx.upload(room)
             ctx.mul_mat(samhip.tensor(12, k, n, wb.ptr + off, nb1=rb), samhip.tensor(samhip.F32, k, m, xb.ptr),
                         samhip.tensor(samhip.F32, n, m, yb.ptr, nb1=4 * ldy))
+            assert (ctx.query().kernel_variant == VARIANT[12]) == (off == 0)
             got = ctx.download(yb, room.shape, np.float32)
             assert row_rel(got[:m, :n], ref) <= (EXACT if off == 0 else 1e-3)
             assert (got[:m, n:] == 3.0).all() and (got[m] == 3.0).all()
@@ -79,6 +83,7 @@ def test_strip16_capture_and_noalloc(samhip, oracle):
         W, X = samhip.tensor(13, k, n, wb.ptr), samhip.tensor(samhip.F32, k, m, xb.ptr)
         Y, Z = samhip.tensor(samhip.F32, n, m, yb.ptr), samhip.tensor(samhip.F32, n, m, zb.ptr)
         ctx.mul_mat(W, X, Y)
+        assert ctx.query().kernel_variant == VARIANT[13]
         eager = ctx.download(yb, (m, n), np.float32)
         samhip.check(samhip.lib().samhip_mul_mat_noalloc(ctx.handle, ctypes.byref(W), ctypes.byref(X), ctypes.byref(Z)))
         assert np.array_equal(ctx.download(zb, (m, n), np.float32).view(np.uint32), eager.view(np.uint32))
@@ -152,14 +157,16 @@ def test_settings_for_the_strip_kernel_reach_it(samhip, oracle, monkeypatch, nam
     w = oracle.quantize(12, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
     x = rng.standard_normal((m, k)).astype(np.float32)
 
-    def run():
+    def run(variant):
         with samhip.Context(0) as ctx:
-            return ctx.matmul(12, w, x).view(np.uint32)
+            y = ctx.matmul(12, w, x)
+            assert ctx.query().kernel_variant == variant
+            return y.view(np.uint32)
 
-    default = run()
+    default = run(VARIANT[12])
     monkeypatch.setenv("SAMHIP_STRIP16", "0")
-    strip = run()
-    assert not np.array_equal(default, strip)   # else the next line says nothing
+    strip = run(b"skinny_i8mfma_q4_k")
+    assert not np.array_equal(default, strip)   # else the last line says nothing
     monkeypatch.delenv("SAMHIP_STRIP16")
     monkeypatch.setenv(name, value)
-    assert np.array_equal(run(), strip)
+    assert np.array_equal(run(b"skinny_i8mfma_q4_k"), strip)
