@@ -723,15 +723,14 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     // Q8_0 rows that are not whole 128-value steps meet the fp16 GEMM with
     // zeros up to the next step, unless that needs staging that a
     // no-allocation or captured call does not have: against the in-loader
-    // decode (gemm_kernel, 128x128 tiles) M = 777, N = 1000, K = 1056 takes
-    // 16.3 us for 30.3, M = 5184, N = 1024, K = 4704 88 for 181.  Grids of at
-    // most nine such tiles stay there although the GEMM would win (M = 300,
-    // N = 259, K = 800: 25.6 against 12.2 us): the reported variant of those
-    // products is part of what the library's tests hold fixed.
+    // decode (gemm_kernel, 128x128 tiles; the same bits) M = 300, N = 259,
+    // K = 800 takes 13.5 us for 26.5, M = 777, N = 1000, K = 1056 16.3 for
+    // 30.3, M = 5184, N = 1024, K = 4704 88 for 181; over 3 to 27 tiles and
+    // K = 160 .. 8224 at least 1.5 times faster (1.3 where each call is waited
+    // for), with rows of x that are not 16-byte aligned too.
     int kp = K;
     bool gemm16 = tall;
-    if (!tall && M > kFusedMaxM && !small_w && !ctx->tall_decode && K % 128 != 0 &&
-        int64_t((M + 127) / 128) * ((N + 127) / 128) > 9) {
+    if (!tall && M > kFusedMaxM && !small_w && !ctx->tall_decode && K % 128 != 0) {
         const int padded = (K + 127) / 128 * 128;
         const size_t need = staging_of(padded, true).bytes;
         if (M >= ctx->tall_m && gemm_f16_supported(M, N, padded, padded, padded) &&

@@ -291,20 +291,26 @@ def test_mul_mat_tall_path_tails(gpu_ctx, f16_ctx, oracle, qtype):
 
 
 @pytest.mark.parametrize("k", [800, 1056])
-def test_mul_mat_tall_k_not_multiple_of_128(gpu_ctx, f16_ctx, oracle, k):
+def test_mul_mat_tall_k_not_multiple_of_128(gpu_ctx, f16_ctx, samhip, oracle, monkeypatch, k):
     """M >= 256 with K % 128 != 0 (only Q8_0 rows can be that wide: the
-    K-quants need K % 256 == 0): the pipelined GEMM does not take it, so the
-    staged activations meet gemm_kernel, which decodes the packed weight
-    while staging it into LDS.  M and N tails, fully compared."""
+    K-quants need K % 256 == 0): the pipelined GEMM takes it with zero columns
+    up to its next step; with SAMHIP_TALL_DECODE=1 the staged activations meet
+    gemm_kernel, which decodes the packed weight while staging it into LDS,
+    with the same bits.  M and N tails, fully compared."""
     say("case mul_mat tall fallback", k)
     rng = np.random.default_rng(31 + k)
     w = oracle.quantize(oracle.Q8_0, (rng.standard_normal((259, k)) * 0.02).astype(np.float32))
     x = rng.standard_normal((300, k)).astype(np.float32)
-    yn = gpu_ctx.matmul(8, w, x)
-    assert gpu_ctx.query().kernel_variant == b"gemm_f16mfma_128x128x32_q8_0"
-    yf = f16_ctx.matmul(8, w, x)
-    assert f16_ctx.query().kernel_variant == b"gemm_f16mfma_128x128x32_q8_0"
+    yn, yf = gpu_ctx.matmul(8, w, x), f16_ctx.matmul(8, w, x)
+    assert gpu_ctx.query().kernel_variant.startswith(b"gemm_f16pipe")
+    assert f16_ctx.query().kernel_variant.startswith(b"gemm_f16pipe")
     _check_product(oracle, 8, w, x, yn, yf, DECODED_TOL)
+    monkeypatch.setenv("SAMHIP_TALL_DECODE", "1")
+    for compute, y in ((samhip.COMPUTE_Q8_NATIVE, yn), (samhip.COMPUTE_F16, yf)):
+        with samhip.Context(0, compute) as ctx:
+            loader = ctx.matmul(8, w, x)
+            assert ctx.query().kernel_variant == b"gemm_f16mfma_128x128x32_q8_0"
+        assert np.array_equal(loader.view(np.uint32), y.view(np.uint32))
 
 
 SKINNY_CASES = [(1, 96, 256), (32, 257, 1024), (33, 300, 512), (64, 64, 256), (65, 33, 256), (201, 256, 512),
