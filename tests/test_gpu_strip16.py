@@ -170,3 +170,20 @@ def test_settings_for_the_strip_kernel_reach_it(samhip, oracle, monkeypatch, nam
     monkeypatch.delenv("SAMHIP_STRIP16")
     monkeypatch.setenv(name, value)
     assert np.array_equal(run(b"skinny_i8mfma_q4_k"), strip)
+
+
+@pytest.mark.parametrize("qtype,m,n,k,taken", [(12, 128, 256, 4096, False), (12, 144, 256, 4096, True),
+                                               (12, 64, 512, 4096, True), (13, 64, 512, 4096, False),
+                                               (13, 32, 1024, 4096, True), (13, 33, 4096, 1024, False),
+                                               (12, 33, 4096, 1024, True), (13, 16, 4736, 1024, True)])
+def test_strip16_where_it_is_faster(samhip, oracle, qtype, m, n, k, taken):
+    """Both sides of the lines of strip16_preferred at half the chip and at K
+    in one launch; exact either way."""
+    print("case strip16 line", qtype, m, n, k, flush=True)
+    rng = np.random.default_rng(m + n + k)
+    w = oracle.quantize(qtype, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    with samhip.Context(0) as ctx:
+        y = ctx.matmul(qtype, w, x)
+        assert ctx.query().kernel_variant == (VARIANT[qtype] if taken else VARIANT[qtype].replace(b"16", b""))
+    assert row_rel(y, oracle.mul_mat_native(qtype, w, x)) <= EXACT
