@@ -120,9 +120,9 @@ struct samhip_context {
     // directly, so the call is one launch and a stream wait (a device flag
     // took a fill before and a copy after it: 15 us more a call)
     int* host_flag = nullptr;
-    // strip16's packed activation rows (kStrip16Bytes, for the context's life):
-    // not part of `staging`, so that which kernel a product runs on follows
-    // from its operands alone, in a capture too
+    // strip16's packed activation rows (kStrip16Bytes, from the first such
+    // product or capture on): not part of `staging`, so that which kernel a
+    // product runs on follows from its operands alone, in a capture too
     void* packed_rows = nullptr;
     // this device's fixed scratch (samhip_mul_mat_noalloc); while such a call
     // runs, `staging` points at it and `no_alloc` forbids growing it
@@ -219,6 +219,11 @@ int ensure_staging(samhip_context* ctx, size_t bytes) {
     ctx->staging_bytes = rounded;
     ctx->info.activation_allocation_peak_bytes =
         std::max<uint64_t>(ctx->info.activation_allocation_peak_bytes, rounded);
+    return SAMHIP_OK;
+}
+
+int ensure_packed_rows(samhip_context* ctx) {
+    if (!ctx->packed_rows) HIP_TRY(hipMalloc(&ctx->packed_rows, kStrip16Bytes), "hipMalloc packed rows");
     return SAMHIP_OK;
 }
 
@@ -348,8 +353,7 @@ int samhip_context_create(const samhip_options* options, samhip_context** out) {
     if (hipSetDevice(o.device) != hipSuccess || hipGetDeviceProperties(&prop, o.device) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc(reinterpret_cast<void**>(&ctx->flag), sizeof(int)) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&ctx->host_flag), sizeof(int), hipHostMallocCoherent) != hipSuccess ||
-        hipMalloc(&ctx->packed_rows, kStrip16Bytes) != hipSuccess) {
+        hipHostMalloc(reinterpret_cast<void**>(&ctx->host_flag), sizeof(int), hipHostMallocCoherent) != hipSuccess) {
         samhip_context_destroy(ctx);
         return fail(SAMHIP_ERR_DEVICE, "HIP context initialization failed");
     }
@@ -588,6 +592,8 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
         const size_t reserve = std::max(parts, size_t(256));
         if (int rc = ensure_staging(ctx, ctx->capturing ? std::min(reserve, strip16_bytes(M, K)) : reserve)) return rc;
         static_assert(kStrip16Bytes <= kNoAllocScratchBytes, "the fixed scratch holds the packed rows");
+        if (!ctx->no_alloc)
+            if (int rc = ensure_packed_rows(ctx)) return rc;
         void* const scratch = ctx->no_alloc ? ctx->staging : ctx->packed_rows;
         const char* variant = strip16_variant(w->type);
         int rc = traced(ctx, "stage_strip_q8_k", w->type, M, N, K, [&]() -> int {
@@ -1594,6 +1600,7 @@ int samhip_capture_begin(samhip_context* ctx) {
     if (ctx->tracing) return fail(SAMHIP_ERR_INVALID_ARGUMENT, "capture_begin: a trace is open");
     if (!ctx->stream) return fail(SAMHIP_ERR_INVALID_ARGUMENT, "capture_begin: the null stream cannot be captured");
     if (int rc = set_device(ctx)) return rc;
+    if (int rc = ensure_packed_rows(ctx)) return rc;   // a captured call cannot allocate it
     HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     ctx->capturing = true;
     return SAMHIP_OK;
