@@ -106,7 +106,9 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const _Float16* __restrict
 
     const int nsteps = K / BK;
     auto global_load = [&](int slot, int step) {
-        const int st = min(step, nsteps - 1);   // past the range: a repeat of the last step, never stored to LDS
+        // past the range: a repeat of the last step, which may reach the LDS
+        // buffer that no later step reads, and no product
+        const int st = min(step, nsteps - 1);
         const u32x4* p = reinterpret_cast<const u32x4*>(a_src + BK * st);
         a_reg[slot][0] = p[0];
         a_reg[slot][1] = p[1];

@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restr
     const int i = lane >> 2;
     // lanes past the last block repeat it; their bytes are not stored
     const int64_t g = min(first + i, blocks - 1);
-    const int64_t r = blocks <= 0xffffffff ? int64_t(uint32_t(g) / uint32_t(nb)) : g / nb;
+    const int64_t r = uint32_t(g) / uint32_t(nb);   // (a launch has at most 2^28 blocks)
     const float* xb = x + r * x_stride + 32 * (g - r * nb) + 8 * (lane & 3);
     floatx8 v;
     if (XVEC) {
