@@ -383,11 +383,12 @@ bool strip16_supported(int wtype, int M, int K, const void* w, int64_t w_stride)
 //     leave the chip idle where K slices do not: M = 200, N = 100, K = 4096
 //     9.9 against 8.7, M = 32, N = 512, K = 4096 8.4 against 7.8;
 //   * just 128 of them past K = 1024, half the CUs, with more than four tiles
-//     of rows (Q5_K: two) where the strip kernel (one_launch:
+//     of rows (Q5_K: one) where the strip kernel (one_launch:
 //     kq_strip_i8_preferred takes the product) has K slices for all CUs:
 //     M = 128, N = 256, K = 4096 Q4_K 9.7 against 9.4, Q5_K 10.2 against 9.6
 //     (M = 144: 10.0 against 11.8, 10.5 against 12.0); M = 64, N = 512 Q4_K
-//     9.1 against 9.4, Q5_K 9.7 each, but waited for 20.5 against 19.8;
+//     9.1 against 9.4, Q5_K 9.7 each, but waited for 20.5 against 19.8, and
+//     M = 32, N = 1024 9.8 against 9.7, waited for 20.4 against 19.8;
 //   * K that the strip kernel takes in one launch without a reduction: up to
 //     K = 768 M = 200, N = 1024 8.7 against 8.2; at K = 1024 Q5_K with more
 //     than one tile of rows, M = 255, N = 1024 10.2 against 10.0, M = 128,
@@ -401,7 +402,7 @@ inline bool strip16_preferred(int wtype, int M, int N, int K, int cus, bool one_
     const int64_t rg = (N + 15) / 16, tiles = (M + 15) / 16;
     const int short_k = wtype == T_Q5_K && tiles > 1 ? 1024 : 768;
     if (one_launch && K <= short_k && 256 * i8_strip_slice_sb(wtype, M, N, K, cus) >= K) return false;
-    if (one_launch && K > 1024 && tiles > (wtype == T_Q5_K ? 2 : 4) && rg * tiles <= 128) return false;
+    if (one_launch && K > 1024 && tiles > (wtype == T_Q5_K ? 1 : 4) && rg * tiles <= 128) return false;
     return rg * tiles >= (K > 1024 ? 128 : 64) && rg * ((tiles + 1) / 2) <= 7 * int64_t(cus);
 }
 size_t strip16_bytes(int M, int K);

@@ -272,17 +272,17 @@ def test_kquant_int8_default_routing(samhip, oracle):
     """By default the K-quant int8 path takes the products whose grid of
     row groups x 32-row blocks x K slices fits one round of the chip's CUs,
     with 1024-wide slices for Q4_K / Q5_K (the decoder's 256x256 products at
-    M = 201 and 33) and 256-wide ones for Q6_K, and with K = 256 those that
-    fit one round with 64 weight rows per workgroup (the decoder's M = 201 FFN
-    expansion to 2048); the text encoder's M = 32 products, past one
-    super-block of K, run exact on the 16-row kernel; the rest (M = 201,
-    N = 4096, K = 256; Q6_K M = 32, N = 4096, K = 1024) stays on the fused
-    kernel."""
+    M = 201 and 33, Q5_K at M = 32, K = 4096) and 256-wide ones for Q6_K, and
+    with K = 256 those that fit one round with 64 weight rows per workgroup
+    (the decoder's M = 201 FFN expansion to 2048); the text encoder's other
+    M = 32 products, past one super-block of K, run exact on the 16-row
+    kernel; the rest (M = 201, N = 4096, K = 256; Q6_K M = 32, N = 4096,
+    K = 1024) stays on the fused kernel."""
     rng = np.random.default_rng(5)
     with samhip.Context(0, samhip.COMPUTE_Q8_NATIVE) as ctx:
         strip, strip16, fused = "skinny_i8mfma_", "skinny_i8mfma16_", "skinny_fused_"
         for qt, m, n, k, kernel in ((oracle.Q4_K, 201, 256, 256, strip), (oracle.Q4_K, 33, 256, 256, strip),
-                                    (oracle.Q4_K, 32, 1024, 1024, strip16), (oracle.Q5_K, 32, 1024, 4096, strip16),
+                                    (oracle.Q4_K, 32, 1024, 1024, strip16), (oracle.Q5_K, 32, 1024, 4096, strip),
                                     (oracle.Q4_K, 201, 2048, 256, strip), (oracle.Q4_K, 201, 4096, 256, fused),
                                     (oracle.Q6_K, 32, 1024, 1024, strip), (oracle.Q6_K, 32, 4096, 1024, fused)):
             w = oracle.quantize(qt, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
