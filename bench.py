@@ -320,7 +320,7 @@ def summarize_profiles(d, commands):
     stats_table("encoder", "Kernel time, SAM 3 vision encoder forward at 1008 px (Q4_K qkv/proj/fc1, Q8_0 fc2; "
                 "8 forwards: 2 warmup, 5 timed, 1 traced)", commands["encoder"],
                 "kernel_stats_vision_encoder_1008px_q4_k.md",
-                note="`quantize_weights_kernel` and `quantize_act_kernel` pack the random-init weights once at set-up; "
+                note="`quantize_weights_kernel` and `quantize_q8_0_kernel` pack the random-init weights once at set-up; "
                      "every other kernel runs 8 times per block (or per image for the prefix and the neck).  Template "
                      "arguments: `prep_kernel<mode, chunks, x86, weight type, pre>` (pre 1 = erf-GELU, 2 = layer "
                      "norm), `gemm_f16_pipe_kernel<BM, BN, BK, stages, waves M, waves N, epilogue, A operand>` "
