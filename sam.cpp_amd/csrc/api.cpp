@@ -1127,7 +1127,7 @@ int samhip_flash_attn(samhip_context* ctx, const float* q, const float* k, const
     if (rc) return rc;
     return traced(ctx, attention_name(splits), T_F32, batches * n, heads * 64, n, [&]() -> int {
         if (!launch_attention(ops, out, int64_t(heads) * 64, int(batches), heads, int(n), splits, att_scratch,
-                              att_bytes, ctx->stream))
+                              att_bytes, ctx->cus, ctx->stream))
             return fail(SAMHIP_ERR_UNSUPPORTED, "flash_attn: no attention launch for this grid");
         HIP_TRY(hipGetLastError(), "attention launch");
         return SAMHIP_OK;
@@ -1221,7 +1221,7 @@ int samhip_vit_block(samhip_context* ctx, const samhip_vit_block_desc* d, float*
         if (rc) return rc;
     }
     rc = traced(ctx, attention_name(splits), T_F32, T, E, per, [&]() -> int {
-        if (!launch_attention(ops, ln, E, int(B), int(H), int(per), splits, att_scratch, att_bytes, ctx->stream))
+        if (!launch_attention(ops, ln, E, int(B), int(H), int(per), splits, att_scratch, att_bytes, ctx->cus, ctx->stream))
             return fail(SAMHIP_ERR_UNSUPPORTED, "vit_block: no attention launch for this grid");
         HIP_TRY(hipGetLastError(), "attention launch");
         return SAMHIP_OK;

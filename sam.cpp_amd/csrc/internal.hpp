@@ -157,7 +157,7 @@ void launch_zero_pad(const AttnOperands& o, int B, int H, int N, hipStream_t str
 int attention_splits(int B, int H, int N, bool precise, int cus, int force);
 size_t attention_scratch_bytes(int B, int H, int N, int S);
 bool launch_attention(const AttnOperands& o, float* out, int64_t ldo, int B, int H, int N, int S, float* scratch,
-                      size_t scratch_bytes, hipStream_t stream);
+                      size_t scratch_bytes, int cus, hipStream_t stream);
 // Patch convolution operands as split fp16: A [T][3*Kp] = [hi | hi | lo] of
 // the image patches, W [E][3*Kp] = [hi | lo | hi] of the kernel rows, so
 // A W^T = hi*hi + hi*lo + lo*hi (F32-accurate); Kp = 3*p*p rounded up to 128.

@@ -236,7 +236,10 @@ constexpr float LOG2E = 1.44269504088896340736f;
 __device__ __forceinline__ int v_swizzle(int r) { return 2 * (r & 3) + ((r >> 2) & 1); }
 
 // LEVEL 0: fp16 operands; 1: split scores; 2: split scores and output.
-template <int QW, int LEVEL>   // waves per workgroup (32 queries each), precision level
+// DEEP: for CUs that hold several workgroups for long (launch_attention): the
+// wave with products to issue goes before those in their softmax, and the
+// pair maximum by a swap of register rows instead of through LDS.
+template <int QW, int LEVEL, bool DEEP>   // waves per workgroup (32 queries each), precision level
 __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, float* __restrict__ out, int64_t ldo,
                                                             int H, int N, int Np, int S, float* __restrict__ part_o,
                                                             float* __restrict__ part_ml) {
@@ -254,16 +257,23 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
     __shared__ __attribute__((aligned(1024))) uint8_t ktile[P][2][TB];
     __shared__ __attribute__((aligned(1024))) uint8_t vtile[PV][VB][TB];
     // grid z = window x key split: split sp takes key tiles [kb0, kb1)
-    // Workgroups are dispatched round-robin over the 8 XCDs: XCD x takes a
-    // contiguous run of (key split, head, query block) triples, query blocks
-    // fastest, so that the query blocks that read the same keys share its L2 (with the
-    // row swap for the pair maximum below: windowed 47.0 -> 45.6 us per block)
-    const int nwg = gridDim.x * gridDim.y * gridDim.z;
-    const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int per = nwg / 8, rem = nwg % 8, xcd = id % 8;
-    const int order = xcd * per + min(xcd, rem) + id / 8;
-    const int qblock = order % gridDim.x, plane = order / gridDim.x;
-    const int h = plane % gridDim.y, bz = plane / gridDim.y, b = bz / S, sp = bz - b * S;
+    // Workgroups are dispatched round-robin over the 8 XCDs.  Where several
+    // query blocks read the same keys, XCD x takes a contiguous run of (key
+    // split, head, query block) triples, query blocks fastest, so that they
+    // share its L2: 9 windows of 576 tokens, 16 heads 68.2 -> 65.7 us with the
+    // operands' packing, one of 577 28.5 -> 26.5, one of 400 22.5 -> 20.7.  Not
+    // with one query block (36 windows of 64 tokens 20.9 -> 22.4) nor with
+    // splits of few keys (1024 tokens, 12 heads 29.8 -> 30.4).
+    int qblock = blockIdx.x, h = blockIdx.y, bz = blockIdx.z;
+    if (gridDim.x > 1 && (S == 1 || DEEP)) {
+        const unsigned nwg = gridDim.x * gridDim.y * gridDim.z;
+        const unsigned id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        const unsigned order = id % 8 * (nwg / 8) + min(id % 8, nwg % 8) + id / 8, plane = order / gridDim.x;
+        qblock = order - plane * gridDim.x;
+        bz = plane / gridDim.y;
+        h = plane - bz * gridDim.y;
+    }
+    const int b = bz / S, sp = bz - b * S;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 31, hh = lane >> 5;
     const int64_t bh = int64_t(b) * H + h;
@@ -346,9 +356,7 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
         floatx16 s0, s1;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s0[r] = s1[r] = 0.f;
-        // the wave with products to issue goes before those in their softmax
-        // (a Q8_0 block with global attention 605 -> 602 us)
-        __builtin_amdgcn_s_setprio(1);
+        if (DEEP) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             // rows li and 32 + li, chunk 2s + hh (same swizzle: (32 + li) & 7 == li & 7)
@@ -368,7 +376,7 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
                 s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qf[P - 1][s], s1, 0, 0, 0);
             }
         }
-        __builtin_amdgcn_s_setprio(0);
+        if (DEEP) __builtin_amdgcn_s_setprio(0);
         // keys past N (only in the last tile)
         const int kbase = kb * 64;
         if (kbase + 64 > N) {
@@ -385,8 +393,12 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
         float mx = -__builtin_inff();
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = __builtin_elementwise_maximum(mx, __builtin_elementwise_maximum(s0[r], s1[r]));
-        const auto mx2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-        mx = __builtin_elementwise_maximum(__uint_as_float(mx2[0]), __uint_as_float(mx2[1]));
+        if (DEEP) {
+            const auto other = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+            mx = __builtin_elementwise_maximum(__uint_as_float(other[0]), __uint_as_float(other[1]));
+        } else {
+            mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 32, 64));
+        }
         // Lazy rescaling: the exponent base mrun only moves when a score
         // exceeds it by more than 8 / log2(e), so the weights stay below 2^8
         // (fp16 keeps its full relative precision there) and most tiles skip
@@ -455,7 +467,7 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
             else wait_vmcnt0();
             __syncthreads();
         }
-        __builtin_amdgcn_s_setprio(1);
+        if (DEEP) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             half8 a0, a1;
@@ -471,7 +483,7 @@ __global__ __launch_bounds__(64 * QW) void attention_kernel(AttnOperands op, flo
                 o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(l1, pf[0][u], o1, 0, 0, 0);
             }
         }
-        __builtin_amdgcn_s_setprio(0);
+        if (DEEP) __builtin_amdgcn_s_setprio(0);
         if (kb + 1 < kb1) {
             wait_vmcnt0();   // this wave's loads of the next tile landed
             __syncthreads();
@@ -644,7 +656,7 @@ size_t attention_scratch_bytes(int B, int H, int N, int S) {
 }
 
 bool launch_attention(const AttnOperands& o, float* out, int64_t ldo, int B, int H, int N, int S, float* scratch,
-                      size_t scratch_bytes, hipStream_t stream) {
+                      size_t scratch_bytes, int cus, hipStream_t stream) {
     const int np = (N + 63) / 64 * 64;
     const bool precise = o.ql && o.kl && o.vl;
     if (S < 1 || int64_t(B) * S > 65535) return false;
@@ -660,12 +672,21 @@ bool launch_attention(const AttnOperands& o, float* out, int64_t ldo, int B, int
     // (splitting the scores alone, level 1, measured 6e-4 relative error per
     // output row at 2.8 ms per SAM 3 image against 5e-6 at 3.9 ms for level 2
     // and 4e-3 at 1.9 ms for level 0)
-    if (precise)
-        hipLaunchKernelGGL((attention_kernel<4, 2>), grid, dim3(256), 0, stream, o, out, ldo, H, N, np, S, part_o,
-                           part_ml);
-    else
-        hipLaunchKernelGGL((attention_kernel<4, 0>), grid, dim3(256), 0, stream, o, out, ldo, H, N, np, S, part_o,
-                           part_ml);
+    // DEEP: more workgroups than CUs, each of at least 20 key tiles.  A block
+    // with 72x72 global attention 577.6 -> 576.5 us from the row swap and 602
+    // from 605 from the priorities, with fp16 operands 424 -> 418; 4096 tokens,
+    // 12 heads 161.8 -> 160.5.  Elsewhere both cost: 577 tokens, 16 heads 26.4
+    // -> 28.2 and 28.4 us, 1500 (192 workgroups) 50.5 -> 54.8 and 56.0, 9
+    // windows of 576 66.8 -> 67.7 and 67.6.
+    const bool deep = int64_t(grid.x) * grid.y * grid.z > cus && (np / 64 + S - 1) / S >= 20;
+#define SAMHIP_ATTENTION(LEVEL, DEEP)                                                                                \
+    hipLaunchKernelGGL((attention_kernel<4, LEVEL, DEEP>), grid, dim3(256), 0, stream, o, out, ldo, H, N, np, S, part_o, \
+                       part_ml)
+    if (precise && deep) SAMHIP_ATTENTION(2, true);
+    else if (precise) SAMHIP_ATTENTION(2, false);
+    else if (deep) SAMHIP_ATTENTION(0, true);
+    else SAMHIP_ATTENTION(0, false);
+#undef SAMHIP_ATTENTION
     if (S > 1) {
         const int64_t n = int64_t(B) * N * H * 16;
         hipLaunchKernelGGL(attention_merge_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream, part_o,

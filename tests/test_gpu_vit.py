@@ -94,6 +94,25 @@ def test_flash_attn_key_splits(samhip, oracle, monkeypatch, splits):
         ctx.close()
 
 
+# either side of the line past which the kernel expects several long-lived
+# workgroups on a CU (more than 256 of them, 20 key tiles each), and orders of
+# workgroups over the XCDs that leave a remainder
+@pytest.mark.parametrize("splits,batches,n,heads", [(1, 1, 1300, 24), (1, 1, 1300, 23), (1, 2, 1280, 13), (1, 2, 1216, 13),
+                                                    (2, 1, 2500, 7), (2, 1, 2400, 7), (1, 3, 150, 5)])
+def test_flash_attn_workgroups_per_cu(samhip, oracle, monkeypatch, splits, batches, n, heads):
+    monkeypatch.setenv("SAMHIP_ATTN_SPLITS", str(splits))
+    rng = np.random.default_rng(n + heads)
+    q, k, v = (rng.standard_normal((batches * n, heads * 64)).astype(np.float32) for _ in range(3))
+    say(f"flash_attn splits={splits} batches={batches} n={n} heads={heads}")
+    with samhip.Context(0) as ctx:
+        got = ctx.flash_attn(q, k, v, batches, heads, 0.125)
+    ref = np.concatenate([oracle.attention(q[b * n:(b + 1) * n], k[b * n:(b + 1) * n], v[b * n:(b + 1) * n],
+                                           heads, 64, 0.125) for b in range(batches)])
+    rel = row_rel(got.reshape(-1, 64), ref.reshape(-1, 64))
+    say(f"  max {rel.max():.3g} median {np.median(rel):.3g}")
+    assert rel.max() < 1e-5 and np.median(rel) < 2e-6
+
+
 @pytest.mark.parametrize("splits", [2, 3, 4])
 def test_vit_block_fp16_attention_key_splits(samhip, oracle, monkeypatch, splits):
     """The fp16-operand attention (attention_type F16) with its keys split
