@@ -731,7 +731,7 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     // no-allocation or captured call does not have: against the in-loader
     // decode (gemm_kernel, 128x128 tiles; the same bits) M = 300, N = 259,
     // K = 800 takes 13.5 us for 26.5, M = 777, N = 1000, K = 1056 16.3 for
-    // 30.3, M = 5184, N = 1024, K = 4704 88 for 181; over 3 to 27 tiles and
+    // 30.3, M = 5184, N = 1024, K = 4704 88 (for 150 at K = 4608); over 3 to 27 tiles and
     // K = 160 .. 8224 at least 1.5 times faster (1.3 where each call is waited
     // for), with rows of x that are not 16-byte aligned too.
     int kp = K;
@@ -808,7 +808,7 @@ int samhip_mul_mat(samhip_context* ctx, const samhip_tensor* w, const samhip_ten
     } else {
         rc = traced(ctx, variant, w->type, M, N, K, [&]() -> int {
             if (!launch_gemm(w->type, a, K, rs, w->data, int64_t(w->nb[1]), static_cast<float*>(y->data),
-                             int64_t(y->nb[1] / 4), M, N, K, ctx->stream))
+                             int64_t(y->nb[1] / 4), M, N, K, ctx->cus, ctx->stream))
                 return fail(SAMHIP_ERR_UNSUPPORTED, "mul_mat: no GEMM kernel for this shape");
             HIP_TRY(hipGetLastError(), "gemm launch");
             return SAMHIP_OK;

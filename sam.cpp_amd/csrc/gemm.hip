@@ -48,14 +48,18 @@ template <> struct StepPiece<T_Q8_0> {
     }
 };
 
-// K steps in flight per thread, in registers.  A tile has its CU to itself
-// when the grid is small, and one step's products (8 MFMAs a wave) are far
-// shorter than the latency of its scattered packed-weight loads: M = 300,
-// N = 259, K = 800 (9 tiles) 35.1 -> 25.6 us with its staging, M = 1000,
-// N = 1000, K = 4064 (64 tiles) 138 -> 77; grids of many tiles are level
-// (M = 20000, N = 3000, K = 800 218 -> 222).
+// K steps in flight per thread, in registers, where every tile has a CU to
+// itself: one step's products (8 MFMAs a wave) are far shorter than the
+// latency of its scattered packed-weight loads.  M = 300, N = 259, K = 1024 (9
+// tiles) with its staging Q8_0 44 -> 31 us, Q4_K 58 -> 45, M = 4096, N = 1024
+// (256 tiles) 55 -> 41 and 69 -> 55.
 template <int WT>
 constexpr int kDepth = WT == T_Q8_0 ? 4 : 2;
+// More tiles than CUs hide one another's loads instead: one step in flight,
+// in at most 128 registers, so that four workgroups fit a CU.  Against the
+// rings (145 .. 172 registers, three): M = 5184, N = 3072, K = 1024 Q8_0 92 ->
+// 82 us, Q5_K 131 -> 118, M = 10000, N = 4736 Q4_K 314 -> 285, Q5_K 366 -> 309,
+// M = 3000, N = 1500, K = 2048 (288 tiles) Q8_0 88 -> 77, Q6_K level at 93.
 
 // Tile order: blocks are dispatched round-robin over the 8 XCDs, so give each
 // XCD a contiguous range of tiles, and walk that range in groups of GROUP_M
@@ -73,14 +77,13 @@ __device__ __forceinline__ void tile_of(int bid, int nblocks, int tiles_m, int t
     tn = within / gm;
 }
 
-template <int WT>
+template <int WT, int DEPTH>
 __global__ __launch_bounds__(256, 2) void gemm_kernel(const _Float16* __restrict__ A, int64_t lda,
                                                       const float* __restrict__ row_scale,
                                                       const uint8_t* __restrict__ W, int64_t w_stride,
                                                       float* __restrict__ Y, int64_t ldy, int M, int N, int K,
                                                       int tiles_m, int tiles_n) {
-    constexpr int DEPTH = kDepth<WT>;
-    static_assert(DEPTH % 2 == 0, "the LDS buffer alternates per step");
+    static_assert(DEPTH == 1 || DEPTH % 2 == 0, "the LDS buffer alternates per step");
     __shared__ _Float16 As[2][BM * LDS_STRIDE];
     __shared__ _Float16 Bs[2][BN * LDS_STRIDE];
 
@@ -125,13 +128,6 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const _Float16* __restrict
         bd[1] = half8{w[8], w[9], w[10], w[11], w[12], w[13], w[14], w[15]};
     };
 
-    // slot i of the register ring holds a step s with s % DEPTH == i
-#pragma unroll
-    for (int i = 0; i < DEPTH; ++i) global_load(i, i);
-    lds_store(0, 0, 0);
-    global_load(0, DEPTH);
-    __syncthreads();
-
     const int frag_row = lane & 31, frag_k = 8 * (lane >> 5);
     auto products = [&](int buf) {
 #pragma unroll
@@ -150,25 +146,43 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(const _Float16* __restrict
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
         }
     };
-    // whole turns of the ring without a branch, so that each wait counts
-    // exactly the loads issued since; then the up to DEPTH - 1 steps left
-    int s0 = 0;
-    for (; s0 + DEPTH <= nsteps; s0 += DEPTH) {
-#pragma unroll
-        for (int u = 0; u < DEPTH; ++u) {
-            const int next = (u + 1) % DEPTH;
-            products(u & 1);
-            lds_store((u & 1) ^ 1, next, min(s0 + u + 1, nsteps - 1));
-            global_load(next, s0 + u + 1 + DEPTH);
+    if constexpr (DEPTH == 1) {
+        global_load(0, 0);
+        lds_store(0, 0, 0);
+        __syncthreads();
+        for (int s = 0; s < nsteps; ++s) {
+            if (s + 1 < nsteps) global_load(0, s + 1);
+            products(s & 1);
+            if (s + 1 < nsteps) lds_store((s & 1) ^ 1, 0, s + 1);
             __syncthreads();
         }
-    }
+    } else {
+        // slot i of the register ring holds a step s with s % DEPTH == i
 #pragma unroll
-    for (int u = 0; u < DEPTH - 1; ++u) {
-        if (s0 + u >= nsteps) break;
-        products(u & 1);
-        if (s0 + u + 1 < nsteps) lds_store((u & 1) ^ 1, u + 1, s0 + u + 1);
+        for (int i = 0; i < DEPTH; ++i) global_load(i, i);
+        lds_store(0, 0, 0);
+        global_load(0, DEPTH);
         __syncthreads();
+        // whole turns of the ring without a branch, so that each wait counts
+        // exactly the loads issued since; then the up to DEPTH - 1 steps left
+        int s0 = 0;
+        for (; s0 + DEPTH <= nsteps; s0 += DEPTH) {
+#pragma unroll
+            for (int u = 0; u < DEPTH; ++u) {
+                const int next = (u + 1) % DEPTH;
+                products(u & 1);
+                lds_store((u & 1) ^ 1, next, min(s0 + u + 1, nsteps - 1));
+                global_load(next, s0 + u + 1 + DEPTH);
+                __syncthreads();
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < DEPTH - 1; ++u) {
+            if (s0 + u >= nsteps) break;
+            products(u & 1);
+            if (s0 + u + 1 < nsteps) lds_store((u & 1) ^ 1, u + 1, s0 + u + 1);
+            __syncthreads();
+        }
     }
 
     // 32x32 accumulator layout: lane l holds column l%32, rows 8*(r/4) + 4*(l/32) + r%4.
@@ -201,13 +215,19 @@ const char* gemm_variant(int wtype) {
 }
 
 const char* launch_gemm(int wtype, const _Float16* a, int64_t lda, const float* row_scale, const void* w,
-                        int64_t w_stride, float* y, int64_t ldy, int M, int N, int K, hipStream_t stream) {
+                        int64_t w_stride, float* y, int64_t ldy, int M, int N, int K, int cus, hipStream_t stream) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const dim3 grid(unsigned(tiles_m * tiles_n)), block(256);
     const uint8_t* wb = static_cast<const uint8_t*>(w);
-#define SAMHIP_GEMM(T)                                                                                             \
-    hipLaunchKernelGGL(gemm_kernel<T>, grid, block, 0, stream, a, lda, row_scale, wb, w_stride, y, ldy, M, N, K, \
-                       tiles_m, tiles_n)
+#define SAMHIP_GEMM(T)                                                                                              \
+    do {                                                                                                            \
+        if (tiles_m * tiles_n <= cus)                                                                               \
+            hipLaunchKernelGGL((gemm_kernel<T, kDepth<T>>), grid, block, 0, stream, a, lda, row_scale, wb, w_stride, \
+                               y, ldy, M, N, K, tiles_m, tiles_n);                                                  \
+        else                                                                                                        \
+            hipLaunchKernelGGL((gemm_kernel<T, 1>), grid, block, 0, stream, a, lda, row_scale, wb, w_stride, y, ldy, \
+                               M, N, K, tiles_m, tiles_n);                                                          \
+    } while (0)
     switch (wtype) {
         case T_Q8_0: SAMHIP_GEMM(T_Q8_0); break;
         case T_Q4_K: SAMHIP_GEMM(T_Q4_K); break;

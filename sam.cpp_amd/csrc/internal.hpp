@@ -229,7 +229,7 @@ const char* gemm_variant(int wtype);
 
 // Returns the kernel variant name, or nullptr for an unsupported type.
 const char* launch_gemm(int wtype, const _Float16* a, int64_t lda, const float* row_scale, const void* w,
-                        int64_t w_stride, float* y, int64_t ldy, int M, int N, int K, hipStream_t stream);
+                        int64_t w_stride, float* y, int64_t ldy, int M, int N, int K, int cus, hipStream_t stream);
 
 // Skinny / medium products (M <= kSkinnyMaxM): weights decoded in registers,
 // one pass over the packed bytes.  Returns the variant name, or nullptr.

@@ -81,3 +81,22 @@ def test_padded_k_at_scratch_limits(samhip, oracle):
             ctx.synchronize()
             assert np.array_equal(ctx.download(yb, (m, n), np.float32).view(np.uint32), ref.view(np.uint32))
         graph.destroy()
+
+
+# SAMHIP_TALL_DECODE=1: a ring of K steps in registers up to a tile per CU
+# (256), one step past that; steps of 32 values fewer than the ring holds, and
+# left over after whole turns of it
+@pytest.mark.parametrize("m,n", [(300, 1031), (2200, 2100)])
+@pytest.mark.parametrize("qtype,k", [(8, 64), (8, 96), (8, 160), (8, 288), (12, 256), (13, 512), (14, 256)])
+def test_in_loader_decode_has_the_bits_of_the_staged_weight(gpu_ctx, samhip, oracle, monkeypatch, qtype, m, n, k):
+    print("case in-loader decode", qtype, m, n, k, flush=True)
+    rng = np.random.default_rng(m + n + k)
+    w = oracle.quantize(qtype, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    y = gpu_ctx.matmul(qtype, w, x)
+    assert gpu_ctx.query().kernel_variant.startswith(b"gemm_f16pipe")
+    monkeypatch.setenv("SAMHIP_TALL_DECODE", "1")
+    with samhip.Context(0) as ctx:
+        z = ctx.matmul(qtype, w, x)
+        assert ctx.query().kernel_variant.startswith(b"gemm_f16mfma_128x128x32")
+    assert np.array_equal(y.view(np.uint32), z.view(np.uint32))
