@@ -383,26 +383,29 @@ bool strip16_supported(int wtype, int M, int K, const void* w, int64_t w_stride)
 //     leave the chip idle where K slices do not: M = 200, N = 100, K = 4096
 //     9.9 against 8.7, M = 32, N = 512, K = 4096 8.4 against 7.8;
 //   * just 128 of them past K = 1024, half the CUs, with more than four tiles
-//     of rows (Q5_K: one) where the strip kernel (one_launch:
-//     kq_strip_i8_preferred takes the product) has K slices for all CUs:
-//     M = 128, N = 256, K = 4096 Q4_K 9.7 against 9.4, Q5_K 10.2 against 9.6
-//     (M = 144: 10.0 against 11.8, 10.5 against 12.0); M = 64, N = 512 Q4_K
-//     9.1 against 9.4, Q5_K 9.7 each, but waited for 20.5 against 19.8, and
-//     M = 32, N = 1024 9.8 against 9.7, waited for 20.4 against 19.8;
+//     of rows (Q5_K: one) where the K slices of the strip kernel (one_launch:
+//     kq_strip_i8_preferred takes the product) are one for every CU, as at K =
+//     2048 and 4096: M = 128, N = 256, K = 4096 Q4_K 9.7 against 9.4, Q5_K 10.2
+//     against 9.6 (M = 144: 10.0 against 11.8, 10.5 against 12.0); M = 64, N =
+//     512 Q4_K 9.1 against 9.4, Q5_K 9.7 each, but waited for 20.5 against
+//     19.8, and M = 32, N = 1024 9.8 against 9.7, waited for 20.4 against 19.8
+//     (K = 4608, where the slices leave CUs idle: 10.0 against 12.5);
 //   * K that the strip kernel takes in one launch without a reduction: up to
 //     K = 768 M = 200, N = 1024 8.7 against 8.2; at K = 1024 Q5_K with more
-//     than one tile of rows, M = 255, N = 1024 10.2 against 10.0, M = 128,
-//     N = 2048 9.8 against 9.9 but waited for 21.1 against 20.4.  (Q4_K there
-//     is 1 .. 8 % faster in a graph, M = 48, N = 4096 9.3 against 9.7, and up
-//     to 3 % slower waited for; one tile of rows, N = 4736, takes 7.1 against
-//     9.1, Q5_K 7.5 against 9.3);
+//     than four tiles of rows, M = 255, N = 1024 10.2 against 10.0, M = 128,
+//     N = 2048 9.8 against 9.9 but waited for 21.1 against 20.4 (M = 33, N =
+//     3072 9.5 against 9.9).  Q4_K there is 1 .. 8 % faster in a graph, M = 48,
+//     N = 4096 9.3 against 9.7, and up to 3 % slower waited for;
 //   * more than seven workgroups of 16 x 32 rows per CU: M = 255, N = 4096,
 //     K = 1024 22.0 against the fused kernel's 18.0 (M = 200: 19.6, 22.8).
 inline bool strip16_preferred(int wtype, int M, int N, int K, int cus, bool one_launch) {
     const int64_t rg = (N + 15) / 16, tiles = (M + 15) / 16;
-    const int short_k = wtype == T_Q5_K && tiles > 1 ? 1024 : 768;
-    if (one_launch && K <= short_k && 256 * i8_strip_slice_sb(wtype, M, N, K, cus) >= K) return false;
-    if (one_launch && K > 1024 && tiles > (wtype == T_Q5_K ? 1 : 4) && rg * tiles <= 128) return false;
+    if (one_launch) {
+        const int slice_k = 256 * i8_strip_slice_sb(wtype, M, N, K, cus);
+        const int64_t strip_wgs = int64_t((N + 31) / 32) * ((M + 31) / 32) * ((K + slice_k - 1) / slice_k);
+        if (slice_k >= K && K <= (wtype == T_Q5_K && tiles > 4 ? 1024 : 768)) return false;
+        if (K > 1024 && rg * tiles <= 128 && tiles > (wtype == T_Q5_K ? 1 : 4) && strip_wgs >= cus) return false;
+    }
     return rg * tiles >= (K > 1024 ? 128 : 64) && rg * ((tiles + 1) / 2) <= 7 * int64_t(cus);
 }
 size_t strip16_bytes(int M, int K);

@@ -175,7 +175,8 @@ def test_settings_for_the_strip_kernel_reach_it(samhip, oracle, monkeypatch, nam
 @pytest.mark.parametrize("qtype,m,n,k,taken", [(12, 128, 256, 4096, False), (12, 144, 256, 4096, True),
                                                (12, 64, 512, 4096, True), (13, 64, 512, 4096, False),
                                                (13, 32, 1024, 4096, False), (12, 32, 1024, 4096, True),
-                                               (13, 16, 2048, 4096, True), (13, 33, 4096, 1024, False),
+                                               (13, 16, 2048, 4096, True), (13, 32, 1024, 4608, True),
+                                               (13, 64, 4096, 1024, True), (13, 65, 2048, 1024, False),
                                                (12, 33, 4096, 1024, True), (13, 16, 4736, 1024, True)])
 def test_strip16_where_it_is_faster(samhip, oracle, qtype, m, n, k, taken):
     """Both sides of the lines of strip16_preferred at half the chip and at K
